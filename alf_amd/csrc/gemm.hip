@@ -12,7 +12,8 @@
 // The host picks the tile shape per launch: at Ndim = 256 a 32 x 32 tiling leaves most of
 // the 256 CUs idle, a 16 x 16 tiling with KS = 4 fills them with a quarter of the per-wave K.
 //
-// This one kernel carries every dense product of the sweep:
+// gemm_tile_kernel takes the same products where the grid fills the device without a K split.
+// These kernels carry every dense product of the sweep:
 //   * hopping wraps  G <- D exp(-dtau T) G exp(dtau T) D^-1       (real T: 2 MFMA/step)
 //   * UDV chain      U <- D exp(-dtau T) U,  U <- exp(-dtau T) conj(D) U
 //   * delayed-update flush  G += X Y^T
@@ -22,6 +23,10 @@
 namespace {
 
 constexpr int NT = 256;
+
+// Every MFMA kernel here is bounded to two waves per SIMD at least (second argument of
+// __launch_bounds__): with 256 registers or fewer the compiler keeps the accumulators in VGPRs,
+// without the bound it puts them in AGPRs and moves them there and back around every K stage.
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -216,7 +221,7 @@ __device__ __forceinline__ void scale_b(const cplx s, E& re, E& im) {
 }
 
 template <bool A_CPLX, bool B_CPLX, int WM, int WN, bool F32>
-__global__ __launch_bounds__(NT) void gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs g) {
   typedef Mma<F32> M;
   typedef typename M::E E;
   constexpr int KS = 4 / (WM * WN);
@@ -329,27 +334,54 @@ __global__ __launch_bounds__(NT) void gemm_kernel(GemmArgs g) {
   }
 }
 
-// Register-blocked 64 x 64 tile for grids with several tiles per CU (batched chains): 4
-// waves in a 2 x 2 arrangement, each wave a 32 x 32 sub-tile held as 2 x 2 MFMA blocks, so
-// every operand fragment read from LDS feeds two blocks and a K stage of 16 carries 4x the
-// MFMA work of the 32 x 32 tile per barrier.  The next stage's global loads are in flight
-// (in registers) while the current stage is multiplied out of LDS.
-template <bool A_CPLX, bool B_CPLX, bool F32, int BK>
-__global__ __launch_bounds__(NT, 2) void gemm_big_kernel(GemmArgs g) {
+// Tile kernel for grids that fill the device (batched chains, large lattices): a workgroup of
+// 2 x 2 waves owns a (32 MB) x (32 NB) complex tile, each wave MB x NB blocks of 16 x 16.
+//
+// What bounds it is the FP64 matrix rate (78.6 TF/s, reached by a loop of independent
+// v_mfma_f64_16x16x4f64 whose accumulators stay in VGPRs), so everything else has to stay out of
+// the K loop: the storage order of both operands and their types are template parameters, edges
+// are clamped addresses instead of branches (a clamped row or column is not stored, a clamped k
+// is selected to zero), and the gather maps and row scales are read one stage ahead of the data
+// they serve.  K stages of 16 go global -> registers -> LDS, double-buffered, one barrier per
+// stage, with the next stage's loads in flight during this stage's products.
+// LDS rows hold one k of the tile, complex entries as (re, im) pairs read by one ds_read_b128;
+// the row pads keep both the k-fastest stores and the fragment reads free of bank conflicts.
+// The fragments enter the MFMA exchanged (opB as its first operand), so that the 16 lanes of a
+// result row run along a column of C: 256-byte segments instead of 64.
+//
+// 256 chains of n = 256, per launch: real x complex wraps 430 -> 326 us (53 TF/s), complex x complex
+// 572 -> 500 us (51 TF/s of issued products); one product of n = 1024 issues at 61 TF/s.  The
+// kernel this replaces chose orders, gathers and edges by branches inside the K stage.  128 x 64
+// tiles, three waves per SIMD and K stages of 32 measured the same or slower.
+//
+// AKF / BKF: k is the fastest index in memory (opA = T, C / opB = N).  With both operands complex
+// the product is three real ones (3M): Ar Br, Ai Bi, (Ar + Ai)(Br + Bi).
+template <bool CPLX, bool F32> struct TileElem;
+template <> struct TileElem<false, false> { typedef double T; };
+template <> struct TileElem<true, false> { typedef double2 T; };
+template <> struct TileElem<false, true> { typedef float T; };
+template <> struct TileElem<true, true> { typedef float2 T; };
+
+template <bool A_CPLX, bool B_CPLX, bool AKF, bool BKF, bool EXTRA, bool F32, int MB, int NB>
+__global__ __launch_bounds__(NT, 2) void gemm_tile_kernel(GemmArgs g) {
   typedef Mma<F32> M;
   typedef typename M::E E;
-  constexpr int TM = 64, TN = 64;
-  __shared__ E As_re[BK][TM + 1];
-  __shared__ E As_im[A_CPLX ? BK : 1][TM + 1];
-  __shared__ E Bs_re[BK][TN + 1];
-  __shared__ E Bs_im[B_CPLX ? BK : 1][TN + 1];
-  __shared__ cplx bsl[BK];
+  typedef typename TileElem<A_CPLX, F32>::T TA;
+  typedef typename TileElem<B_CPLX, F32>::T TB;
+  typedef typename TileElem<A_CPLX, false>::T GA;          // elements in memory
+  typedef typename TileElem<B_CPLX, false>::T GB;
+  constexpr int TM = 32 * MB, TN = 32 * NB, BK = 16;
+  constexpr int LA = TM * BK / NT, LB = TN * BK / NT;     // elements per thread and stage
+  // row pitch in elements: an odd number of 16-byte units for the 16-byte rows; for 8-byte rows
+  // 16 entries more than a multiple of 32, so the two k rows of a half-wave read meet other banks
+  constexpr int PA = A_CPLX ? TM + 1 : TM + (AKF ? 2 : 16), PB = B_CPLX ? TN + 1 : TN + (BKF ? 2 : 16);
+  __shared__ __align__(16) TA As[2][BK][PA];
+  __shared__ __align__(16) TB Bs[2][BK][PB];
 
   const int tid = threadIdx.x;
   int bx, by, bz;
   xcd_order(bx, by, bz);
-  const int i0 = bx * TM;
-  const int j0 = by * TN;
+  const int i0 = bx * TM, j0 = by * TN;
   if (chain_operands(g, bz)) { identity_tile(g, i0, j0, TM, TN, tid, blockDim.x); return; }
   const int z = bz % (g.batch > 1 ? g.batch : 1);
   int K = g.K;
@@ -358,115 +390,207 @@ __global__ __launch_bounds__(NT, 2) void gemm_big_kernel(GemmArgs g) {
     K = kd < K ? kd : K;
   }
   if (K <= 0 && g.beta.x == 1.0 && g.beta.y == 0.0) return;  // nothing to add
-
-  const long long za = g.batch > 1 ? z * g.strideA : 0, zb = g.batch > 1 ? z * g.strideB : 0;
-  const void* A = A_CPLX ? (const void*)((const cplx*)g.A + za) : (const void*)((const double*)g.A + za);
-  const void* B = g.b_cplx ? (const void*)((const cplx*)g.B + zb) : (const void*)((const double*)g.B + zb);
+  const GA* const A = (const GA*)g.A + (g.batch > 1 ? z * g.strideA : 0);
+  const GB* const B = (const GB*)g.B + (g.batch > 1 ? z * g.strideB : 0);
   cplx* C = (cplx*)g.C + (g.batch > 1 ? z * g.strideC : 0);
+  // the row scales of opB multiply opB, or the columns of opA when only opA is complex
+  constexpr bool SCALE_A = A_CPLX && !B_CPLX;
+  const double ca = g.opA == OP_C ? -1.0 : 1.0, cb = g.opB == OP_C ? -1.0 : 1.0;
+
+  // this thread's elements of a stage: k offset and tile index of element p
+  auto a_k = [&](int p) { return AKF ? tid % BK : (tid + NT * p) / TM; };
+  auto a_i = [&](int p) { return AKF ? tid / BK + (NT / BK) * p : (tid + NT * p) % TM; };
+  auto b_k = [&](int p) { return BKF ? tid % BK : (tid + NT * p) / TN; };
+  auto b_j = [&](int p) { return BKF ? tid / BK + (NT / BK) * p : (tid + NT * p) % TN; };
+  constexpr int KA = AKF ? 1 : LA, KB = BKF ? 1 : LB;     // distinct k of a thread per stage
+  const int kmax = K > 0 ? K - 1 : 0;
+  auto clampk = [&](int k) { return k < kmax ? k : kmax; };
+  // element offsets inside a stage; the stage's own offset k0 is added to the uniform base
+  // pointer, so a full stage costs no address arithmetic (tile_kernel_takes keeps them in 32 bits)
+  unsigned ao[LA], bo[LB];
+#pragma unroll
+  for (int p = 0; p < LA; ++p) {
+    const int i = i0 + a_i(p) < g.M ? i0 + a_i(p) : g.M - 1;
+    ao[p] = AKF ? (unsigned)i * (unsigned)g.lda : (unsigned)i;
+    if (!EXTRA) ao[p] += AKF ? (unsigned)a_k(p) : (unsigned)a_k(p) * (unsigned)g.lda;
+  }
+#pragma unroll
+  for (int p = 0; p < LB; ++p) {
+    const int j = j0 + b_j(p) < g.N ? j0 + b_j(p) : g.N - 1;
+    bo[p] = BKF ? (unsigned)j * (unsigned)g.ldb : (unsigned)j;
+    if (!EXTRA) bo[p] += BKF ? (unsigned)b_k(p) : (unsigned)b_k(p) * (unsigned)g.ldb;
+  }
+  // EXTRA: gathered k of the next stage's elements, read one stage ahead
+  unsigned ka[EXTRA ? KA : 1], kb[EXTRA ? KB : 1];
+  auto load_k = [&](int k0) {
+    if constexpr (EXTRA) {
+#pragma unroll
+      for (int p = 0; p < KA; ++p) { const int k = clampk(k0 + a_k(p)); ka[p] = g.amap ? g.amap[k] : k; }
+#pragma unroll
+      for (int p = 0; p < KB; ++p) { const int k = clampk(k0 + b_k(p)); kb[p] = g.bmap ? g.bmap[k] : k; }
+    }
+  };
+  GA av[LA];
+  GB bv[LB];
+  cplx sv[EXTRA ? (SCALE_A ? KA : KB) : 1];
+  auto load = [&](int k0) {
+    if constexpr (EXTRA) {
+#pragma unroll
+      for (int p = 0; p < LA; ++p) {
+        const unsigned k = ka[AKF ? 0 : p];
+        av[p] = A[AKF ? ao[p] + k : ao[p] + k * (unsigned)g.lda];
+      }
+#pragma unroll
+      for (int p = 0; p < LB; ++p) {
+        const unsigned k = kb[BKF ? 0 : p];
+        bv[p] = B[BKF ? bo[p] + k : bo[p] + k * (unsigned)g.ldb];
+      }
+      if (g.bs) {
+#pragma unroll
+        for (int p = 0; p < (SCALE_A ? KA : KB); ++p) sv[p] = g.bs[clampk(k0 + (SCALE_A ? a_k(p) : b_k(p)))];
+      }
+    } else {
+      const GA* const Ak = A + (AKF ? (long long)k0 : (long long)k0 * g.lda);
+      const GB* const Bk = B + (BKF ? (long long)k0 : (long long)k0 * g.ldb);
+      if (k0 + BK <= K) {
+#pragma unroll
+        for (int p = 0; p < LA; ++p) av[p] = Ak[ao[p]];
+#pragma unroll
+        for (int p = 0; p < LB; ++p) bv[p] = Bk[bo[p]];
+      } else {
+        const int kl = kmax - k0;                         // last k of the partial stage
+#pragma unroll
+        for (int p = 0; p < LA; ++p) {
+          const unsigned over = a_k(p) > kl ? a_k(p) - kl : 0;
+          av[p] = Ak[ao[p] - (AKF ? over : over * (unsigned)g.lda)];
+        }
+#pragma unroll
+        for (int p = 0; p < LB; ++p) {
+          const unsigned over = b_k(p) > kl ? b_k(p) - kl : 0;
+          bv[p] = Bk[bo[p] - (BKF ? over : over * (unsigned)g.ldb)];
+        }
+      }
+    }
+  };
+  auto store = [&](int k0, int buf) {
+    if (k0 + BK > K) {
+      // the partial last stage: elements beyond K are zero
+#pragma unroll
+      for (int p = 0; p < LA; ++p)
+        if (k0 + a_k(p) >= K) av[p] = GA{};
+#pragma unroll
+      for (int p = 0; p < LB; ++p)
+        if (k0 + b_k(p) >= K) bv[p] = GB{};
+    }
+#pragma unroll
+    for (int p = 0; p < LA; ++p) {
+      if constexpr (A_CPLX) {
+        cplx v = av[p];
+        if (AKF) v.y *= ca;
+        if constexpr (EXTRA && SCALE_A) if (g.bs) v = cmul(v, sv[AKF ? 0 : p]);
+        As[buf][a_k(p)][a_i(p)] = TA{(E)v.x, (E)v.y};
+      } else {
+        As[buf][a_k(p)][a_i(p)] = (E)av[p];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < LB; ++p) {
+      if constexpr (B_CPLX) {
+        cplx v = bv[p];
+        if (!BKF) v.y *= cb;
+        if constexpr (EXTRA && !SCALE_A) if (g.bs) v = cmul(v, sv[BKF ? 0 : p]);
+        Bs[buf][b_k(p)][b_j(p)] = TB{(E)v.x, (E)v.y};
+      } else {
+        Bs[buf][b_k(p)][b_j(p)] = (E)bv[p];
+      }
+    }
+  };
 
   const int wave = tid >> 6, lane = tid & 63;
-  const int wr = 32 * (wave & 1), wc = 32 * (wave >> 1);
   const int lr = lane & 15, lk = lane >> 4;
-
-  // complex x complex in three real products (3M): acc_re = Ar Br, acc_t2 = Ai Bi,
-  // acc_im = (Ar + Ai)(Br + Bi); re = acc_re - acc_t2, im = acc_im - acc_re - acc_t2
+  const int wr = 16 * MB * (wave & 1), wc = 16 * NB * (wave >> 1);
   constexpr bool M3 = A_CPLX && B_CPLX;
-  typename M::Acc acc_re[2][2], acc_im[2][2], acc_t2[M3 ? 2 : 1][M3 ? 2 : 1];
+  typename M::Acc acc_re[MB][NB], acc_im[MB][NB], acc_t2[M3 ? MB : 1][M3 ? NB : 1];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < MB; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < NB; ++b) {
       acc_re[a][b] = typename M::Acc{0, 0, 0, 0};
       acc_im[a][b] = typename M::Acc{0, 0, 0, 0};
       if (M3) acc_t2[M3 ? a : 0][M3 ? b : 0] = typename M::Acc{0, 0, 0, 0};
     }
 
-  Stage<TM, TN, BK, A_CPLX, B_CPLX> st;
-
-  if (K > 0) st.load(g, A, B, i0, j0, K, 0, tid);
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    st.store(g, tid, As_re, As_im, Bs_re, Bs_im, bsl);
+  if (K > 0) {
+    load_k(0);
+    load(0);
+    load_k(BK);
+  }
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
+    store(k0, buf);
     __syncthreads();
-    if (k0 + BK < K) st.load(g, A, B, i0, j0, K, k0 + BK, tid);
+    if (k0 + BK < K) {
+      load(k0 + BK);
+      load_k(k0 + 2 * BK);
+    }
+    // the fragments of the next k-step are read while this one's products issue (left to itself
+    // the compiler waits for every k-step's reads in front of its first product)
+    TA fa[2][MB];
+    TB fb[2][NB];
+    auto frag = [&](int kq) {
+#pragma unroll
+      for (int a = 0; a < MB; ++a) fa[(kq >> 2) & 1][a] = As[buf][kq + lk][wr + 16 * a + lr];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) fb[(kq >> 2) & 1][b] = Bs[buf][kq + lk][wc + 16 * b + lr];
+    };
+    frag(0);
 #pragma unroll
     for (int kq = 0; kq < BK; kq += 4) {
-      const int kk = kq + lk;
-      E a_re[2], a_im[2], b_re[2], b_im[2];
+      const int f = (kq >> 2) & 1;
+      if (kq + 4 < BK) frag(kq + 4);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        a_re[a] = As_re[kk][wr + 16 * a + lr];
-        if (A_CPLX) a_im[a] = As_im[kk][wr + 16 * a + lr];
-      }
+      for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        b_re[b] = Bs_re[kk][wc + 16 * b + lr];
-        if (B_CPLX) b_im[b] = Bs_im[kk][wc + 16 * b + lr];
-      }
-      if (B_CPLX && g.bs) {
-        const cplx sk = bsl[kk];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) scale_b(sk, b_re[b], b_im[b]);
-      }
-      if (M3) {
-        E as[2], bsum[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) as[a] = a_re[a] + a_im[a];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) bsum[b] = b_re[b] + b_im[b];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            acc_re[a][b] = M::mac(a_re[a], b_re[b], acc_re[a][b]);
-            acc_t2[M3 ? a : 0][M3 ? b : 0] = M::mac(a_im[a], b_im[b], acc_t2[M3 ? a : 0][M3 ? b : 0]);
-            acc_im[a][b] = M::mac(as[a], bsum[b], acc_im[a][b]);
+        for (int b = 0; b < NB; ++b) {
+          if constexpr (M3) {
+            acc_re[a][b] = M::mac(fb[f][b].x, fa[f][a].x, acc_re[a][b]);
+            acc_t2[a][b] = M::mac(fb[f][b].y, fa[f][a].y, acc_t2[a][b]);
+            acc_im[a][b] = M::mac(fb[f][b].x + fb[f][b].y, fa[f][a].x + fa[f][a].y, acc_im[a][b]);
+          } else if constexpr (B_CPLX) {
+            acc_re[a][b] = M::mac(fb[f][b].x, fa[f][a], acc_re[a][b]);
+            acc_im[a][b] = M::mac(fb[f][b].y, fa[f][a], acc_im[a][b]);
+          } else {
+            acc_re[a][b] = M::mac(fb[f][b], fa[f][a].x, acc_re[a][b]);
+            acc_im[a][b] = M::mac(fb[f][b], fa[f][a].y, acc_im[a][b]);
           }
-      } else {
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            acc_re[a][b] = M::mac(a_re[a], b_re[b], acc_re[a][b]);
-            if (B_CPLX) acc_im[a][b] = M::mac(a_re[a], b_im[b], acc_im[a][b]);
-          }
-        if (A_CPLX) {
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc_im[a][b] = M::mac(a_im[a], b_re[b], acc_im[a][b]);
         }
-      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-  }
-  if (M3) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const typename M::Acc t2 = acc_t2[M3 ? a : 0][M3 ? b : 0];
-        acc_im[a][b] = acc_im[a][b] - acc_re[a][b] - t2;
-        acc_re[a][b] = acc_re[a][b] - t2;
-      }
   }
 
-  // register r of a lane holds row M::row(r, lane / 16) of its 16 x 16 block
+  // register r of a lane holds column M::row(r, lane / 16) and row lane % 16 of its block
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int gj = j0 + wc + 16 * b + lr;
-    if (gj >= g.N) continue;
-    const cplx csj = g.cs ? g.cs[gj] : make_double2(1.0, 0.0);
+  for (int a = 0; a < MB; ++a) {
+    const int gi = i0 + wr + 16 * a + lr;
+    if (gi >= g.M) continue;
+    cplx rsi = g.rs ? g.rs[gi] : make_double2(1.0, 0.0);
+    if (g.rs_real) rsi = cscale(rsi, g.rs_real[gi]);
+    rsi = cmul(g.alpha, rsi);
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int b = 0; b < NB; ++b) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gi = i0 + wr + 16 * a + M::row(r, lk);
-        if (gi >= g.M) continue;
-        cplx v = make_double2(acc_re[a][b][r], (A_CPLX || B_CPLX) ? acc_im[a][b][r] : 0.0);
-        v = cmul(g.alpha, v);
-        if (g.rs) v = cmul(g.rs[gi], v);
-        if (g.rs_real) v = cscale(v, g.rs_real[gi]);
-        if (g.cs) v = cmul(v, csj);
+        const int gj = j0 + wc + 16 * b + M::row(r, lk);
+        if (gj >= g.N) continue;
+        double re = acc_re[a][b][r], im = acc_im[a][b][r];
+        if constexpr (M3) {
+          const double t2 = acc_t2[a][b][r];
+          im = im - re - t2;
+          re = re - t2;
+        }
+        cplx v = cmul(rsi, make_double2(re, im));
+        if (g.cs) v = cmul(v, g.cs[gj]);
         const long long off = gi + (long long)gj * g.ldc;
         if (g.beta.x != 0.0 || g.beta.y != 0.0) v = cadd(v, cmul(g.beta, C[off]));
         C[off] = v;
@@ -595,25 +719,37 @@ void launch_shape(const GemmArgs& g, hipStream_t s) {
   else launch_shape_p<WM, WN, false>(g, s);
 }
 
-template <bool F32, int BK>
-void launch_big_p(const GemmArgs& g, hipStream_t s) {
-  dim3 grid((unsigned)cdivl(g.M, 64), (unsigned)cdivl(g.N, 64), gemm_zdim(g));
-  const bool bc = g.b_cplx || g.bs != nullptr;
-  // complex x complex always in K stages of 16 (32 would not fit two waves per SIMD)
-  if (g.a_cplx && bc) hipLaunchKernelGGL((gemm_big_kernel<true, true, F32, 16>), grid, dim3(NT), 0, s, g);
-  else if (g.a_cplx) hipLaunchKernelGGL((gemm_big_kernel<true, false, F32, BK>), grid, dim3(NT), 0, s, g);
-  else if (bc) hipLaunchKernelGGL((gemm_big_kernel<false, true, F32, BK>), grid, dim3(NT), 0, s, g);
-  else hipLaunchKernelGGL((gemm_big_kernel<false, false, F32, BK>), grid, dim3(NT), 0, s, g);
+// The tile kernel takes every product with exactly one or two complex operands whose elements
+// are addressable with 32-bit offsets; FP32 operands only in the order of the hopping wraps (N x N).
+bool tile_kernel_takes(const GemmArgs& g) {
+  if (!g.a_cplx && !g.b_cplx) return false;
+  const long long ea = (long long)g.lda * (g.opA == OP_N ? g.K : g.M), eb = (long long)g.ldb * (g.opB == OP_N ? g.N : g.K);
+  if (ea >= (1LL << 27) || eb >= (1LL << 27)) return false;
+  return !g.prec || (g.opA == OP_N && g.opB == OP_N);
 }
-// K stages of 32 for long products with a real operand (the hopping and UDV wraps): twice
-// the MFMA work per barrier and per load latency; complex x complex stays at 16, where 32
-// would not fit two waves per SIMD without spilling
-void launch_big(const GemmArgs& g, hipStream_t s) {
-  const bool deep = g.K >= 64 && !(g.a_cplx && (g.b_cplx || g.bs != nullptr));
-  if (g.prec) deep ? launch_big_p<true, 32>(g, s) : launch_big_p<true, 16>(g, s);
-  else deep ? launch_big_p<false, 32>(g, s) : launch_big_p<false, 16>(g, s);
+template <bool A_CPLX, bool B_CPLX, bool AKF, bool BKF, bool F32, int MB, int NB>
+void launch_tile_o(const GemmArgs& g, hipStream_t s) {
+  dim3 grid((unsigned)cdivl(g.M, 32 * MB), (unsigned)cdivl(g.N, 32 * NB), gemm_zdim(g));
+  if (g.bs || g.amap || g.bmap)
+    hipLaunchKernelGGL((gemm_tile_kernel<A_CPLX, B_CPLX, AKF, BKF, true, F32, MB, NB>), grid, dim3(NT), 0, s, g);
+  else
+    hipLaunchKernelGGL((gemm_tile_kernel<A_CPLX, B_CPLX, AKF, BKF, false, F32, MB, NB>), grid, dim3(NT), 0, s, g);
 }
-
+template <bool A_CPLX, bool B_CPLX, int MB, int NB>
+void launch_tile_p(const GemmArgs& g, hipStream_t s) {
+  const bool akf = g.opA != OP_N, bkf = g.opB == OP_N;
+  if (g.prec) launch_tile_o<A_CPLX, B_CPLX, false, true, true, MB, NB>(g, s);
+  else if (akf && bkf) launch_tile_o<A_CPLX, B_CPLX, true, true, false, MB, NB>(g, s);
+  else if (akf) launch_tile_o<A_CPLX, B_CPLX, true, false, false, MB, NB>(g, s);
+  else if (bkf) launch_tile_o<A_CPLX, B_CPLX, false, true, false, MB, NB>(g, s);
+  else launch_tile_o<A_CPLX, B_CPLX, false, false, false, MB, NB>(g, s);
+}
+template <int MB, int NB>
+void launch_tile(const GemmArgs& g, hipStream_t s) {
+  if (g.a_cplx && g.b_cplx) launch_tile_p<true, true, MB, NB>(g, s);
+  else if (g.a_cplx) launch_tile_p<true, false, MB, NB>(g, s);
+  else launch_tile_p<false, true, MB, NB>(g, s);
+}
 
 // Direct-load split-K kernel for grids that would not fill the device: a workgroup of
 // NW waves owns one 16 x 16 output tile; wave w takes the w-th contiguous quarter
@@ -622,7 +758,7 @@ void launch_big(const GemmArgs& g, hipStream_t s) {
 // four or eight k-steps per batch with the next batch in flight.  The NW partial tiles are
 // summed through LDS in wave order.
 template <bool A_CPLX, bool B_CPLX, int NW, bool F32>
-__global__ __launch_bounds__(64 * NW) void gemm_direct_kernel(GemmArgs g) {
+__global__ __launch_bounds__(64 * NW, 2) void gemm_direct_kernel(GemmArgs g) {
   typedef Mma<F32> M;
   typedef typename M::E E;
   __shared__ cplx red[NW > 1 ? NW - 1 : 1][256];
@@ -810,7 +946,7 @@ void launch_direct(const GemmArgs& g, hipStream_t s) {
 // then the waves split the rank-m product over k and add their halves through LDS.  Every
 // global load of the tile is issued before the first MFMA.
 constexpr int RF_T = 16;
-__global__ __launch_bounds__(128) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
+__global__ __launch_bounds__(128, 2) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
                                                           const cplx* __restrict__ W, const int* __restrict__ amap,
                                                           const int* mdev, int n, int kmax, long long cs) {
   typedef Mma<false> M;
@@ -997,14 +1133,18 @@ int gemm_launch(const GemmArgs& g, hipStream_t s) {
   {
     // two or more 64 x 64 tiles per CU, at least 3/4 of each tile's area inside the product
     const long long tm = cdivl(g.M, 64), tn = cdivl(g.N, 64);
-    if (tm * tn * b >= tile_policy(g).big_from && 4LL * g.M * g.N >= 3LL * (64 * tm) * (64 * tn)) {
-      launch_big(g, s);
+    if (tm * tn * b >= tile_policy(g).big_from && 4LL * g.M * g.N >= 3LL * (64 * tm) * (64 * tn) &&
+        tile_kernel_takes(g)) {
+      launch_tile<2, 2>(g, s);
       HIP_OK(hipGetLastError());
       return ST_NONE;
     }
   }
   switch (gemm_tile_shape(g.M, g.N, g.K, (int)gemm_zdim(g))) {
-    case 0: launch_shape<2, 2>(g, s); break;
+    case 0:
+      if (tile_kernel_takes(g)) launch_tile<1, 1>(g, s);
+      else launch_shape<2, 2>(g, s);
+      break;
     case 1: launch_shape<1, 2>(g, s); break;
     default: launch_shape<1, 1>(g, s); break;
   }
