@@ -175,7 +175,6 @@ __global__ void chain_reset_kernel(ChainState* st, long long cs) {
   st = chain_ptr(st, cs);
   st->pos = 0;
   st->m = 0;
-  st->rng_slice_base = st->rng_pos;
 }
 
 inline unsigned nblk(long long count, int per) { return (unsigned)((count + per - 1) / per); }
@@ -306,13 +305,15 @@ struct alfq_ctx {
   unsigned long long seed = 0;
   unsigned stream_id = 0;
   long long per_visit_sum = 0;           // uniforms per pass over all ops
+  BVisit* vrec = nullptr;                // visit records of a pass, n_op per slice
+  bool multi_op = false;                 // some site has several operators
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   KTimer chain_timer;
   int rounds = 1 << 30;                  // chain rounds per slice (adapted per sweep)
   bool round_fusion = true;              // one launch for a round's X product and flush (few chains)
   int* stat_dev = nullptr;               // 3 words per chain read after every sweep
   int* stat_host = nullptr;              // their pinned host copy
-  bool uniforms_ready = false;           // a whole sweep's uniforms are already on the device
+  bool visits_ready = false;             // the visits of the running pass are prepared
   // sweeps replayed as HIP graphs, keyed by the host state they start from
   struct HostState {
     cplx* G; cplx* Gtmp; double* u;
@@ -416,6 +417,22 @@ int fill_uniforms(alfq_ctx* c, long long count) {
   return launch_philox_fill(c->u, c->st, count, c->B, c->cs, c->s);
 }
 
+// What the Metropolis visits of slices [s0, s0 + ns) of a pass need before they start: the block
+// kernel's visit records, or the uniforms of the generic kernel.
+int prepare_visits(alfq_ctx* c, int s0, int ns, int dir) {
+  if (c->rng_mode == 0 || chain_max_delay(c->n) < c->K) return fill_uniforms(c, ns * c->per_visit_sum);
+  VisitArgs a{};
+  a.out = c->vrec; a.st = c->st; a.f = c->f;
+  a.u = c->rng_mode == 1 ? c->u : nullptr;
+  a.op_site = c->op_site; a.op_type = c->op_type;
+  a.uoff = dir > 0 ? c->uoff_up : c->uoff_dn;
+  a.op_myexp = c->myexp; a.op_expalpha = c->expalpha; a.gama_ratio = c->gama_ratio;
+  a.lz = c->lz;
+  a.n_op = c->n_op; a.s0 = s0; a.ns = ns; a.dir = dir; a.per = (int)c->per_visit_sum;
+  a.cs = c->cs; a.nchain = c->B;
+  return launch_visits(a, c->s);
+}
+
 int metropolis_slice(alfq_ctx* c, int slice, int dir) {
   int st;
   ChainArgs a{};
@@ -429,6 +446,9 @@ int metropolis_slice(alfq_ctx* c, int slice, int dir) {
   a.cs = c->cs; a.nchain = c->B;
   a.lz = c->lz;
   a.uoff = dir > 0 ? c->uoff_up : c->uoff_dn;
+  a.rec = c->vrec + (long long)slice * c->n_op;
+  a.per = (int)c->per_visit_sum;
+  a.multi = c->multi_op ? 1 : 0;
   const int worst = c->n_op / c->K + 1;
   const bool reg_kernel = chain_max_delay(c->n) >= c->K;
   int rounds = worst;
@@ -695,7 +715,7 @@ int wrapgrup_dev(alfq_ctx* c, int ntau) {
     if ((st = gemm_c(c, g2))) return st;
   }
   std::swap(c->G, c->Gtmp);
-  if (!c->uniforms_ready && (st = fill_uniforms(c, c->per_visit_sum))) return st;
+  if (!c->visits_ready && (st = prepare_visits(c, slice, 1, +1))) return st;
   return metropolis_slice(c, slice, +1);
 }
 
@@ -703,7 +723,7 @@ int wrapgrdo_dev(alfq_ctx* c, int ntau) {
   int st;
   if ((st = hop_ready(c))) return st;
   const int slice = ntau - 1;
-  if (!c->uniforms_ready && (st = fill_uniforms(c, c->per_visit_sum))) return st;
+  if (!c->visits_ready && (st = prepare_visits(c, slice, 1, -1))) return st;
   if ((st = metropolis_slice(c, slice, -1))) return st;
   if ((st = launch_dvec(c->f, c->n_op, slice, 1, c->n, c->site_ptr, c->site_ops, c->eexp, c->dv_d, c->dv_dinv,
                         c->dv_dconj, c->B, c->cs, c->s)))
@@ -969,12 +989,9 @@ int init_dev(alfq_ctx* c) {
 
 int sweep_dev(alfq_ctx* c) {
   int st;
-  const auto& s = c->stab;
-  const int L = c->L;
-  if ((st = fill_uniforms(c, 2LL * L * c->per_visit_sum))) return st;
-  c->uniforms_ready = true;
+  c->visits_ready = true;
   st = sweep_body(c);
-  c->uniforms_ready = false;
+  c->visits_ready = false;
   return st;
 }
 
@@ -1015,6 +1032,7 @@ int sweep_body(alfq_ctx* c) {
   int st;
   const auto& s = c->stab;
   const int L = c->L;
+  if ((st = prepare_visits(c, 0, L, +1))) return st;
   if ((st = udv_reset_dev(c, &c->var_r, 'R'))) return st;
   int nst = 1;
   for (int ntau = 0; ntau < L; ++ntau) {
@@ -1030,6 +1048,7 @@ int sweep_body(alfq_ctx* c) {
     }
     if ((st = measure_dev(c, ntau1))) return st;          // main.F90:757-772
   }
+  if ((st = prepare_visits(c, 0, L, -1))) return st;
   if ((st = udv_reset_dev(c, &c->var_l, 'L'))) return st;
   nst = c->nstm - 1;
   for (int ntau = L; ntau >= 1; --ntau) {
@@ -1309,6 +1328,7 @@ void place_chain(alfq_ctx* c, ArenaLayout& ar, int nslot) {
   c->Yc = ar.take<cplx>(nn);
   c->cscal = ar.take<cplx>(4 * (size_t)n);
   c->u_arena = ar.take<double>((size_t)std::max<long long>(c->u_cap, 1));
+  c->vrec = ar.take<BVisit>((size_t)no * c->L);
   qr_work_place(c->qr, n, ar);
   c->pool.assign(nslot, UDVSlot{});
   for (auto& sl : c->pool) {
@@ -1378,7 +1398,10 @@ int create_impl(const alfq_model_desc* descs, int nchain, alfq_ctx** out) {
     typ[i] = d->op_type[i];
     sptr[site[i] + 1] += 1;
   }
-  for (int i = 0; i < n; ++i) sptr[i + 1] += sptr[i];
+  for (int i = 0; i < n; ++i) {
+    c->multi_op = c->multi_op || sptr[i + 1] > 1;
+    sptr[i + 1] += sptr[i];
+  }
   {
     std::vector<int> fillp(sptr.begin(), sptr.end() - 1);
     for (int i = 0; i < no; ++i) sops[fillp[site[i]]++] = i;

@@ -6,7 +6,8 @@
 #include <vector>
 
 #define CHAIN_KMAX 64   // largest delayed-update depth
-#define CHAIN_W_LD 32   // leading dimension of the block kernel's W
+#define CHAIN_BLOCK_KMAX 32   // largest delayed-update depth of the block kernel
+#define CHAIN_W_LD 64   // leading dimension of the block kernel's W
 
 // Per-chain device state touched by the sequential Metropolis kernel.
 struct ChainState {
@@ -17,7 +18,6 @@ struct ChainState {
   int m;                          // pending delayed updates in X/Y
   int status;                     // 1: random stream exhausted
   int pad;
-  unsigned long long rng_slice_base;  // rng_pos at the start of the current slice
   int slice_acc;                  // accepted flips in the current slice
   int max_slice_acc;              // largest slice_acc seen since the host last cleared it
   unsigned long long u_base;      // global index of u[0] in the uniform buffer
@@ -26,6 +26,21 @@ struct ChainState {
   unsigned stream;                // Philox stream of this chain
   int pad2;
 };
+
+// One visit of the block kernel: proposal, table entries and random numbers, prepared for a whole
+// pass (or one slice) by launch_visits.  With Delta = exp(Z1 E) - 1 the single-colour ratio is
+// exp(Z1 alpha) (exp(Z1 E) - Delta G(P,P)) = ca - cb G(P,P); the Metropolis test
+// |Re(PHASE ratio^N_SUN Gama(new)/Gama(old))| / |Re(PHASE)| > u becomes
+// |Re(z ratio^N_SUN)| > thr |Re(z)| with thr = u / |Gama ratio| and z any positive
+// multiple of PHASE, so the decision needs no division.
+struct BVisit {
+  cplx ca, cb, delta;
+  double thr;
+  int P;                    // site
+  short fnew;               // proposed field value; VISIT_NONE: no random numbers left for this visit
+  short loc;                // (kernel) index of the site in its block, the site's first visit there
+};
+#define VISIT_NONE 127
 
 struct ChainArgs {
   cplx* G; int n;
@@ -38,10 +53,13 @@ struct ChainArgs {
   int n_sun;
   const double* u;                // uniforms u[q - st->u_base], q in [st->u_base, st->u_base + st->u_len)
   const int* uoff;                // uniforms consumed before visit v of the slice (n_op + 1 entries)
+  const BVisit* rec;              // block kernel: the slice's n_op visits in order (per chain)
+  int per;                        // uniforms of a whole slice, uoff[n_op]
+  int multi;                      // nonzero: some site has several operators
   int first_round;                // start of the slice: visit 0, rng base = current position
   int final_round;                // last scheduled round: flush in place instead of stopping at K
   ChainState* st;
-  // block kernel outputs for the flush G += (G(:, amap) W) Y^T: W (32 x 32, ld 32), site list
+  // block kernel outputs for the flush G += (G(:, amap) W) Y^T: W (ld CHAIN_W_LD), site list
   cplx* W; int* amap;
   // nonzero: the round's X = G(:, amap) W product writes Yhat (GemmArgs::yhat), so the block
   // kernel leaves Y alone except in its own in-place flush
@@ -67,6 +85,25 @@ struct KTimer {
 int launch_chain(const ChainArgs& a, hipStream_t s, KTimer* timer = nullptr);
 // largest delay depth the submatrix block kernel supports (deeper delays use the generic kernel)
 int chain_max_delay(int n);
+// Visit records of slices [s0, s0 + ns) in the order of a pass (dir > 0: ascending slices and
+// operators) into out[slice * n_op + v], the random numbers taken from st->rng_pos on: from u (a
+// tape, u[q - st->u_base]) or, with u null, from the chain's Philox stream.  A field changes only at
+// its own visit, so the records of a pass do not depend on its decisions.  Tables, f, st and out
+// per chain; lz as in ChainArgs.
+struct VisitArgs {
+  BVisit* out;
+  const ChainState* st;
+  const int8_t* f;
+  const double* u;
+  const int *op_site, *op_type, *uoff;
+  const cplx *op_myexp, *op_expalpha;
+  const double* gama_ratio;
+  const int* lz;
+  int n_op, s0, ns, dir, per;
+  long long cs;
+  int nchain;
+};
+int launch_visits(const VisitArgs& a, hipStream_t s);
 // uniforms of global indices [st->rng_pos, st->rng_pos + count) into u with the chain's
 // Philox key and stream (st->seed, st->stream); records the window in st
 int launch_philox_fill(double* u, ChainState* st, long long count, int nchain, long long cs, hipStream_t s);

@@ -181,11 +181,11 @@ constexpr int GEMM_POLICIES = 4;
 // true when gemm_launch runs g on the direct-load kernel (the only one that honours yhat)
 bool gemm_direct_path(const GemmArgs& g);
 // G += X Y^T (all n x n / n x m, column-major, ld n) with the rank m read from *mdev and
-// clamped to kmax <= 32, for the nchain chains of a batch (pointers advance by cs bytes).
+// clamped to kmax <= CHAIN_BLOCK_KMAX, for the nchain chains of a batch (pointers advance by cs bytes).
 int flush_launch(cplx* G, const cplx* X, const cplx* Y, const int* mdev, int n, int kmax, int nchain,
                  long long cs, hipStream_t s);
 // the round's X product and flush in one launch for a few chains: Go = Gi + (Gi(:, A) W) Yhat^T
-// with Yhat(c, j) = delta(c, amap[j]) - Gi(amap[j], c), rank m = *mdev <= kmax <= 32; W is
-// m x m with leading dimension 32; Gi and Go are different buffers.
+// with Yhat(c, j) = delta(c, amap[j]) - Gi(amap[j], c), rank m = *mdev <= kmax <= CHAIN_BLOCK_KMAX; W is
+// m x m with leading dimension CHAIN_W_LD; Gi and Go are different buffers.
 int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* W, const int* amap, const int* mdev, int n, int kmax,
                        int nchain, long long cs, hipStream_t s);

@@ -46,6 +46,13 @@ __device__ inline uint4 philox4x32_10(uint4 c, uint2 k) {
   return c;
 }
 
+// uniform number q of a chain's Philox stream (the value philox_fill_kernel leaves at q)
+__device__ inline double philox_uniform(unsigned long long q, unsigned long long seed, unsigned stream) {
+  const uint4 r = philox4x32_10(make_uint4((uint32_t)q, (uint32_t)(q >> 32), stream, 0x414c4651u),
+                                make_uint2((uint32_t)seed, (uint32_t)(seed >> 32)));
+  return (double)((((uint64_t)r.x << 32) | r.y) >> 11) * (1.0 / 9007199254740992.0);
+}
+
 // uniforms u[q - base] for global indices q in [base, base + count), base = st->rng_pos: one
 // Philox block per index, 53-bit mantissa from two words, u in [0, 1).  The window is read
 // from and recorded in device memory, so a captured sweep replays with the stream's position.
@@ -60,12 +67,7 @@ __global__ void philox_fill_kernel(double* __restrict__ u, ChainState* st, long 
     st->u_len = count;
   }
   if (i >= count) return;
-  const unsigned long long q = base + (unsigned long long)i;
-  const uint4 c = make_uint4((uint32_t)q, (uint32_t)(q >> 32), stream, 0x414c4651u);
-  const uint2 k = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
-  const uint4 r = philox4x32_10(c, k);
-  const uint64_t w = ((uint64_t)r.x << 32) | r.y;
-  u[i] = (double)(w >> 11) * (1.0 / 9007199254740992.0);
+  u[i] = philox_uniform(base + (unsigned long long)i, seed, stream);
 }
 
 __device__ inline cplx wave_csum(cplx v) {
@@ -92,6 +94,64 @@ __device__ inline int flip_st(int s, int k) {
     case 1: return k == 1 ? 2 : (k == 2 ? -2 : -1);
     default: return k == 1 ? -2 : (k == 2 ? -1 : 1);
   }
+}
+
+// One thread per visit (VisitArgs).  The block kernel would otherwise look a visit up itself, four
+// dependent loads deep, each a miss in the caches a new kernel starts with: 2.9 us of a launch for
+// one chain, 11 us in a batch of 256, against one load of 64 bytes.
+__global__ void visit_kernel(VisitArgs a) {
+  a.out = chain_ptr(a.out, a.cs);
+  a.st = chain_ptr(a.st, a.cs);
+  a.f = chain_ptr(a.f, a.cs);
+  a.u = chain_ptr(a.u, a.cs);
+  a.op_myexp = chain_ptr(a.op_myexp, a.cs);
+  a.op_expalpha = chain_ptr(a.op_expalpha, a.cs);
+  a.gama_ratio = chain_ptr(a.gama_ratio, a.cs);
+  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (long long)a.n_op * a.ns) return;
+  const int v = (int)(idx % a.n_op), q = (int)(idx / a.n_op);
+  const int slice = a.dir > 0 ? a.s0 + q : a.s0 + a.ns - 1 - q;
+  int ord = q;               // slices of the pass that the chain has visited before this one
+  if (a.lz) {
+    const int lz = a.lz[blockIdx.z], end = a.s0 + a.ns;
+    if (slice >= lz) return;
+    if (a.dir < 0 && lz < end) ord -= end - lz;
+  }
+  const int nop = a.dir > 0 ? v : a.n_op - 1 - v;
+  const int typ = a.op_type[nop];
+  const int s_old = a.f[(long long)slice * a.n_op + nop];
+  const int need = a.uoff[v + 1] - a.uoff[v];
+  const unsigned long long pos = a.st->rng_pos + (unsigned long long)ord * a.per + a.uoff[v];
+  BVisit w;
+  w.ca = make_double2(1.0, 0.0); w.cb = make_double2(0.0, 0.0); w.delta = make_double2(0.0, 0.0);
+  w.thr = 2.0; w.fnew = VISIT_NONE; w.loc = 0;
+  w.P = a.op_site[nop];
+  double u0 = 0.0, u1 = 0.0;  // the proposal's number (type 2) and the decision's
+  bool ok = true;
+  if (a.u) {
+    const unsigned long long ub = a.st->u_base;
+    ok = !(pos < ub || pos + (unsigned long long)need > ub + (unsigned long long)a.st->u_len);
+    if (ok) {
+      u0 = a.u[pos - ub];
+      u1 = a.u[pos - ub + need - 1];
+    }
+  } else {
+    const unsigned long long seed = a.st->seed;
+    const unsigned stream = a.st->stream;
+    if (typ == 2) u0 = philox_uniform(pos, seed, stream);
+    u1 = philox_uniform(pos + need - 1, seed, stream);
+  }
+  if (ok) {
+    const int s_new = typ == 2 ? flip_st(s_old, nranf3(u0)) : -s_old;
+    const int ti = nop * 25 + (s_old + 2) * 5 + (s_new + 2);
+    const cplx myexp = a.op_myexp[ti], expal = a.op_expalpha[ti];
+    w.delta = make_double2(myexp.x - 1.0, myexp.y);
+    w.ca = cmul(expal, myexp);
+    w.cb = cmul(expal, w.delta);
+    w.thr = u1 / fabs(a.gama_ratio[ti]);
+    w.fnew = (short)s_new;
+  }
+  a.out[(long long)slice * a.n_op + v] = w;
 }
 
 __global__ __launch_bounds__(256) void chain_kernel(ChainArgs a) {
@@ -203,42 +263,45 @@ __global__ __launch_bounds__(256) void chain_kernel(ChainArgs a) {
 // ---------------------------------------------------------------------------------
 // Submatrix block kernel.  The visits of a round are taken in blocks of up to SB_V
 // consecutive visits.  For the sites S of a block the kernel holds g = G_cur[S, S] in
-// LDS and decides each visit from g alone (G_cur(P,P) = g(p,p)); every thread computes
-// the decision itself, so a rejected proposal needs no barrier and no global load.
-// An accepted flip is the rank-1 update of upgrade_mod.F90:266-269 restricted to S,
-//   g += u w^T,  u = -x g(:, p),  w = e_p - g(p, :)^T,
-// and u, w are the restrictions to S of the delayed-update columns X(:, j), Y(:, j).
+// LDS and decides each visit from g alone (G_cur(P,P) = g(p,p)).  An accepted flip is the
+// rank-1 update of upgrade_mod.F90:266-269 restricted to S,
+//   g += u w^T,  u = -x g(:, p),  w = e_p - g(p, :)^T.
 //
-// The full columns are never formed one flip at a time.  With A = (P_0, P_1, ...) the
-// sites of the round's accepted flips in order and G the Green's function at the start
-// of the round,
-//   X = G(:, A) C,   Y = Yhat D,   Yhat(:, j) = e_{P_j} - G(P_j, :)^T,
-//   C(:, j) = -x_j (e_j + sum_{i<j} C(:, i) Y(P_j, i)),
-//   D(:, j) =        e_j - sum_{i<j} D(:, i) X(P_j, i),
-// with C, D upper triangular of the round's size; the entries X(P_j, i), Y(P_j, i)
-// are already in LDS (u, w of the block, or the block-start rows below).  A block
-// starts from X[S, :] = G[S, A] C, Y[S, :] = Yhat[S, :] D and
-// g = G[S, S] + X[S, :] Y[S, :]^T.  At the end of the round the kernel leaves
-// W = C D^T, the site list A and Yhat; the flush is G += (G(:, A) W) Yhat^T, two GEMMs
-// over the whole device.  All round-sized tables are kept zero outside the round's
-// m x m corner, so their sums run in unconditional groups of four.
+// Full columns and rows of G are never formed here.  With A = (P_0, P_1, ...) the sites of
+// the round's accepted flips in order, G the Green's function at the start of the round and
+// Yhat(:, j) = e_{P_j} - G(P_j, :)^T, the current one is G_cur = G + G(:, A) W Yhat^T with
+// W m x m.  A block of flips extends W to W + Cn Dn^T, whose new columns are
+//   Cn(:, j) = -x_j (e_j + T2(:, p_j) + sum_{i<j} Cn(:, i) w_i(p_j)),   T2 = W Yhat[S]^T,
+//   Dn(:, j) =        e_j - T1(p_j, :)^T - sum_{i<j} Dn(:, i) u_i(p_j), T1 = G[S, A] W
+// (i, j over the block's flips), and the block starts from g = G[S, S] + T1 Yhat[S]^T.  T1, T2,
+// g and the update of W are on the matrix cores, and W is the only table that the round keeps.
+// W's tiles stay in the accumulators of the waves that own them; for T1 and T2 they are copied to
+// LDS, over the tables of the visits.  At the end the kernel leaves W and the site list A; the
+// flush is G += (G(:, A) W) Yhat^T over the device.
+//
+// What bounds it: the chain of decisions, so the instructions and waits per accepted flip.  One
+// wave decides (no barrier inside a block), left-looking: lanes 0..31 hold column p of g, lanes
+// 32..63 row p, each formed from the block-start g and the block's earlier u_i, w_i in LDS, so a
+// flip costs one LDS round trip and a dot product over the block's flips instead of an update of
+// all of g by four waves between barriers; lane v keeps g(v, v) of its visit.  Two more waves
+// follow it flip by flip through flags in LDS and form the columns Cn and Dn (row l of W in
+// lane l), and a fourth fetches the next block's visit records, so that a block ends when its
+// last decision does.
 constexpr int SB_V = 32;    // visits per block: g is SB_V x SB_V
 constexpr int SB_A = 16;    // accepted flips per block
-constexpr int SB_K = 32;    // accepted flips per round (delayed-update depth)
-constexpr int SB_R = 256;   // visit records prepared at once
-static_assert(SB_K == CHAIN_W_LD, "W is stored with the round's size as leading dimension");
+constexpr int SB_K = CHAIN_BLOCK_KMAX;   // accepted flips per round (delayed-update depth)
+constexpr int SB_T = 512;   // threads: 8 waves, two MFMA streams per SIMD
+constexpr int SB_W = SB_T / 64;
+constexpr int SB_M = (SB_K + 15) / 16;   // 16-wide tiles of W
+constexpr int SB_PS = SB_V + 1;          // row pitch of the tables indexed by the block's sites
+constexpr int SB_PW = SB_K + 1;          // row pitch of W
+constexpr int SB_PL = SB_K + 1;          // row pitch of Cn, Dn (index l of W)
+constexpr int SB_TW = (SB_M * SB_M + SB_W - 1) / SB_W;   // tiles of W per wave
+static_assert((2 * SB_A - 1) * SB_PL + 16 * SB_M <= SB_K * SB_PS, "Cn and Dn lie over Yhat[S, A]");
+static_assert(SB_K <= CHAIN_W_LD, "W is stored with CHAIN_W_LD as leading dimension");
+static_assert(SB_K % 4 == 0 && 16 * SB_M <= 64, "row l of Cn and Dn is lane l of a wave");
 
-// One visit.  With Delta = exp(Z1 E) - 1 the single-colour ratio is
-// exp(Z1 alpha) (exp(Z1 E) - Delta G(P,P)) = ca - cb G(P,P); the Metropolis test
-// |Re(PHASE ratio^N_SUN Gama(new)/Gama(old))| / |Re(PHASE)| > u becomes
-// |Re(z ratio^N_SUN)| > thr |Re(z)| with thr = u / |Gama ratio| and z any positive
-// multiple of PHASE, so the decision needs no division.
-struct BVisit {
-  cplx ca, cb, delta;
-  double thr;
-  int loc;                  // index of the site in its block (the site's first visit there)
-  int P;                    // site
-};
+typedef double v4d __attribute__((ext_vector_type(4)));
 
 // z * 2^-e with |z| in [0.5, 1): an exact rescaling that keeps the running phase in range
 __device__ __forceinline__ cplx renorm_pow2(cplx z) {
@@ -257,41 +320,94 @@ __device__ __forceinline__ cplx lane_c(cplx v, int l) {
   return make_double2(__builtin_bit_cast(double, r), __builtin_bit_cast(double, i));
 }
 
-__device__ __forceinline__ void block_sync_lds() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __asm__ volatile("" ::: "memory");
+// lanes 0..31 of v in both halves of low, lanes 32..63 in both halves of high (register moves)
+__device__ __forceinline__ void both_halves(double v, double& low, double& high) {
+  const long long b = __double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)(b & 0xffffffffLL), (unsigned)(b & 0xffffffffLL), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  low = __longlong_as_double(((long long)hi[0] << 32) | (long long)lo[0]);
+  high = __longlong_as_double(((long long)hi[1] << 32) | (long long)lo[1]);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void chain_block_kernel(ChainArgs a) {
-  static_assert(SB_V == 32 && SB_K == 32 && SB_A == 16 && SB_R == 256, "layout of the block kernel");
-  __shared__ cplx gs[2][SB_V * SB_V];              // g(r, c) at [r + SB_V c]; gs[1] also stages G[S, A]
-  __shared__ cplx Xb[SB_K][SB_V], Yb[SB_K][SB_V];  // X(P_s, i), Y(P_s, i) of the round's earlier flips
-  __shared__ cplx UW[2 * SB_A * SB_V];             // u_j(s), w_j(s) of the block's flips; also stages Yhat[S, A]
-  __shared__ cplx Cm[SB_K][SB_K], Dm[SB_K][SB_K];  // C(l, j) at Cm[j][l], D(l, j) at Dm[j][l]
-  __shared__ BVisit vr[SB_R];                      // visits [vbase, vbase + SB_R)
-  __shared__ int2 vaux[SB_R];                      // (proposed field, operator)
-  __shared__ cplx s_x[SB_K];
-  __shared__ int s_aP[SB_K], s_aloc[SB_A];
-  __shared__ int s_pos0, s_stop;
-  __shared__ unsigned long long s_base, s_ubase;
-  __shared__ long long s_ulen;
-  __shared__ cplx s_phase;
-  __shared__ long long s_nc, s_accn;
-  cplx* const Us = UW;
-  cplx* const Ws = UW + SB_A * SB_V;
+// A 16 x 16 complex tile in three real accumulations: re = r - t, im = i - r - t
+struct Tile3 {
+  v4d r = {0, 0, 0, 0}, i = {0, 0, 0, 0}, t = {0, 0, 0, 0};
+  __device__ __forceinline__ void mac(cplx a, cplx b) {
+    r = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, r, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, t, 0, 0, 0);
+    i = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x + a.y, b.x + b.y, i, 0, 0, 0);
+  }
+  __device__ __forceinline__ cplx get(int q) const { return make_double2(r[q] - t[q], i[q] - r[q] - t[q]); }
+};
+// tile += sum over k < kn (a multiple of 4) of fa(k + lk) fb(k + lk), lk = lane / 16: the next
+// step's operands are read while this step's products issue.  Register q of a lane holds the
+// entry of fa's index 4 q + lane / 16 and fb's index lane % 16.
+template <class FA, class FB>
+__device__ __forceinline__ void tile_mac(Tile3& c, int kn, int lk, FA fa, FB fb) {
+  if (kn <= 0) return;
+  cplx a = fa(lk), b = fb(lk);
+  for (int k = 4; k < kn; k += 4) {
+    const cplx an = fa(k + lk), bn = fb(k + lk);
+    c.mac(a, b);
+    a = an;
+    b = bn;
+  }
+  c.mac(a, b);
+}
 
-  const int tid = threadIdx.x;
+// the value of v, which the compiler takes for a new one: address arithmetic made from it stays
+// inside the loop that it is in, where it would otherwise be hoisted, held in registers over the
+// whole loop and spilled
+__device__ __forceinline__ int here(int v) {
+  __asm__ volatile("" : "+v"(v));
+  return v;
+}
+
+// orders LDS accesses in the program; a wave's own LDS operations complete in that order
+__device__ __forceinline__ void lds_order() { __asm__ volatile("" ::: "memory"); }
+
+// Bound by the serial chain of decisions: about 1240 clocks from one acceptance to the next (LDS
+// reads of the row and column, their dot product, the test, the ballot), 20 to 32 of them in a
+// launch.  Per launch for one chain of 16 x 16 22.8 us, where one rank-1 update of X, Y and g per
+// acceptance took 30.4 (its sweep 74.9 -> 65.0 ms); for 256 chains of 16 x 16 42.9 -> 38.7 us, of
+// 4 x 4 20.0 -> 14.3 us.  Rounds deeper than 32 lose in T1, T2 and W what they save in launches
+// (one chain's sweep at 40, 48 and 56: +2, +3 and +7 %).
+// No array of this kernel may leave the registers: one that the compiler moves to LDS by thread
+// costs a read of the launch packet in host memory, 1.6 us and in a batch of 256 chains 8 us.
+__global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
+  // W(l, j) at Wm[l][j] for T1 and T2; during the visits g(r, c) at gs[c][r] and u_i(s), w_i(s)
+  // at Tuw[i][s], Tuw[i][32 + s]
+  __shared__ cplx s_u[SB_K * SB_PW > SB_V * SB_PS + SB_A * 64 ? SB_K * SB_PW : SB_V * SB_PS + SB_A * 64];
+  cplx(*const Wm)[SB_PW] = (cplx(*)[SB_PW])s_u;
+  cplx(*const gs)[SB_PS] = (cplx(*)[SB_PS])s_u;
+  cplx(*const Tuw)[64] = (cplx(*)[64])(s_u + SB_V * SB_PS);
+  __shared__ cplx Xa[SB_K][SB_PS];            // G(S_s, A_l) at [l][s], then T1(s, l)
+  __shared__ cplx Yh[SB_K][SB_PS];            // Yhat(S_s, l) at [l][s]; during the visits Cn, Dn
+  __shared__ cplx Wy[SB_K][SB_PS];            // T2(l, s) at [l][s]
+  __shared__ BVisit vr[2][SB_V];
+  __shared__ cplx s_x[SB_A];
+  __shared__ int s_aP[SB_K];
+  __shared__ int s_mb, s_k, s_stopped;
+  // entry j: 1 + the index of flip j's site once flip j is in LDS, SB_FIN after the block's last
+  __shared__ int s_pub[SB_A + 1];
+  constexpr int SB_FIN = 0x100;
+  cplx* const Cn = &Yh[0][0];                 // Cn(l, j) at Cn[j * SB_PL + l], Dn alike
+  cplx* const Dn = Cn + SB_A * SB_PL;
+
+  // (a wave's LDS operations complete in program order)
+  auto publish = [&](int j, int what) {
+    lds_order();
+    __hip_atomic_store(&s_pub[j], what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lr = lane & 15, lk = lane >> 4;
   const int n = a.n;
-  const int ga = tid & (SB_V - 1), gq = tid >> 5;   // g entries (ga, gq + 8 q), q = 0..3
   a.G = chain_ptr(a.G, a.cs);
   a.X = chain_ptr(a.X, a.cs);
   a.Y = chain_ptr(a.Y, a.cs);
   a.f = chain_ptr(a.f, a.cs);
-  a.op_myexp = chain_ptr(a.op_myexp, a.cs);
-  a.op_expalpha = chain_ptr(a.op_expalpha, a.cs);
-  a.gama_ratio = chain_ptr(a.gama_ratio, a.cs);
-  a.u = chain_ptr(a.u, a.cs);
+  a.rec = chain_ptr(a.rec, a.cs);
   a.st = chain_ptr(a.st, a.cs);
   a.W = chain_ptr(a.W, a.cs);
   a.amap = chain_ptr(a.amap, a.cs);
@@ -301,118 +417,421 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     if (tid == 0) st->m = 0;
     return;
   }
+  // one lane reads the chain's state for the workgroup, with what it will need at the end
+  __shared__ int s_pos0;
+  __shared__ cplx s_phase;
+  ChainState st0;
   if (tid == 0) {
+    st0.nc = st->nc;
+    st0.acc = st->acc;
+    st0.rng_pos = st->rng_pos;
+    st0.max_slice_acc = st->max_slice_acc;
+    st0.slice_acc = a.first_round ? 0 : st->slice_acc;
     s_pos0 = a.first_round ? 0 : st->pos;
-    s_base = a.first_round ? st->rng_pos : st->rng_slice_base;
     s_phase = st->phase;
-    s_nc = st->nc;
-    s_accn = st->acc;
-    s_ubase = st->u_base;
-    s_ulen = st->u_len;
-    if (a.first_round) st->slice_acc = 0;
   }
   __syncthreads();
-  const unsigned long long base = s_base, u_base = s_ubase;
-  const long long u_len = s_ulen;
+  if (s_pos0 >= a.n_op) {
+    // the slice ended in an earlier round
+    if (tid == 0) st->m = 0;
+    return;
+  }
   int pos = s_pos0, m = 0;
-  cplx z = s_phase;         // the phase up to a positive factor
+  cplx z = s_phase;           // the phase up to a positive factor (wave 0)
   long long nvisits = 0, naccepts = 0;
   const int kmax = a.Kmax < SB_K ? a.Kmax : SB_K;
-  int vbase = 0, stop_at = a.n_op;
-  bool have_records = false, stopped = false;
+  bool stopped = false;
 
-  auto zero_cd = [&]() {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      Cm[gq + 8 * q][ga] = make_double2(0.0, 0.0);
-      Dm[gq + 8 * q][ga] = make_double2(0.0, 0.0);
-    }
-  };
-  // records of visits [vbase, vbase + SB_R): proposal, table entries, uniforms (a field
-  // changes only at its own visit, so these do not depend on earlier decisions)
-  auto build_records = [&]() {
-    if (tid == 0) s_stop = a.n_op;
-    __syncthreads();
-    const int v = vbase + tid;
+  // ---- the records of visits v0 .. v0 + SB_V - 1, one per lane of one wave ----
+  auto records = [&](int v0, int buf) {
+    const int lane = here(tid & 63);
     BVisit w;
     w.ca = make_double2(1.0, 0.0); w.cb = make_double2(0.0, 0.0); w.delta = make_double2(0.0, 0.0);
-    w.thr = 2.0; w.P = 0; w.loc = 0;
-    int2 ax = make_int2(0, 0);
-    if (v < a.n_op) {
-      const int nop = a.dir > 0 ? v : a.n_op - 1 - v;
-      const int typ = a.op_type[nop];
-      const int s_old = a.f[(long long)a.slice * a.n_op + nop];
-      const unsigned long long q = base + (unsigned long long)a.uoff[v];
-      const unsigned long long need = (unsigned long long)(a.uoff[v + 1] - a.uoff[v]);
-      const bool ok = !(q < u_base || q + need > u_base + (unsigned long long)u_len);
-      int s_new = -s_old;
-      double u3 = 2.0;
-      if (ok) {
-        const double* u = a.u + (q - u_base);
-        if (typ == 2) { s_new = flip_st(s_old, nranf3(u[0])); u3 = u[2]; } else { u3 = u[1]; }
-      } else {
-        atomicMin(&s_stop, v);
+    w.thr = 2.0; w.P = 0; w.fnew = VISIT_NONE;
+    if (lane < SB_V && v0 + lane < a.n_op) w = a.rec[v0 + lane];
+    w.loc = (short)lane;
+    if (a.multi) {
+      for (int t = 0; t < SB_V; ++t) {
+        const int Pt = __builtin_amdgcn_readlane(w.P, t);
+        if (t < w.loc && Pt == w.P) w.loc = (short)t;
       }
-      const int ti = nop * 25 + (s_old + 2) * 5 + (s_new + 2);
-      const cplx myexp = a.op_myexp[ti], expal = a.op_expalpha[ti];
-      w.delta = make_double2(myexp.x - 1.0, myexp.y);
-      w.ca = cmul(expal, myexp);
-      w.cb = cmul(expal, w.delta);
-      w.thr = u3 / fabs(a.gama_ratio[ti]);
-      w.P = a.op_site[nop];
-      ax = make_int2(s_new, nop);
     }
-    vr[tid] = w;
-    vaux[tid] = ax;
-    __syncthreads();
-    stop_at = s_stop;
-    have_records = true;
+    if (lane < SB_V) vr[buf][lane] = w;
   };
-  // W = C D^T into gs[1] (zero outside m x m): W(l, j) = sum_i C(l, i) D(j, i)
-  // Column j of C and D is zero for j >= m, so of a thread's columns gq + 8 q only q < live_q(m)
-  // can be nonzero in a product with them (the same bound for every lane of the wave).  The
-  // products below are instantiated per bound (with_count), so their loops stay unrolled with
-  // every load of a step issued ahead of its FMAs.
-  auto live_q = [&](int mm) {
-    const int q = (mm - 2 * (tid >> 6) + 7) >> 3;
-    return __builtin_amdgcn_readfirstlane(q < 0 ? 0 : (q > 4 ? 4 : q));
-  };
-  auto with_count = [](int c, auto&& f) {
-    switch (c) {
-      case 1: f(std::integral_constant<int, 1>{}); break;
-      case 2: f(std::integral_constant<int, 2>{}); break;
-      case 3: f(std::integral_constant<int, 3>{}); break;
-      case 4: f(std::integral_constant<int, 4>{}); break;
-      default: break;
+
+  // ---- G at the sites of a block and of the round's flips, in registers until the tables of
+  // the block before are free ----
+  constexpr int NE = (SB_V * SB_K + SB_T - 1) / SB_T;
+  auto gather = [&](const BVisit* v, int nb, cplx (&gss)[4], cplx (&gsa)[NE], cplx (&gas)[NE]) {
+    const int ln = here(lane), lr = ln & 15, lk = ln >> 4, td = here(tid);
+    if (wave < 4) {
+      // tile wave of G[S, S] in the layout of its product: rows lane % 16, columns 4 q + lane / 16
+      const int r = 16 * (wave & 1) + lr;
+      const long long Pr = v[r < nb ? r : 0].P;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = 16 * (wave >> 1) + 4 * q + lk;
+        gss[q] = a.G[Pr + (long long)v[c < nb ? c : 0].P * n];
+      }
+    }
+    const int s = td & (SB_V - 1), Ps = v[s < nb ? s : 0].P;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int l = (td >> 5) + (SB_T / SB_V) * e;
+      if (l < m) {
+        const int Pl = s_aP[l];
+        // (by components: as a copy of the element the array would leave the registers)
+        const cplx *const psa = a.G + Ps + (long long)Pl * n, *const pas = a.G + Pl + (long long)Ps * n;
+        gsa[e] = make_double2(psa->x, psa->y);
+        gas[e] = make_double2(pas->x, pas->y);
+      }
     }
   };
-  auto form_w = [&]() {
-    cplx acc[4];
+  // this wave's tiles of W, (tl, tj) = (t % SB_M, t / SB_M) for t = wave, wave + SB_W, ..: register
+  // q of a lane holds row 16 tl + 4 q + lane / 16 and column 16 tj + lane % 16; zero outside m x m
+  cplx wt[SB_TW][4];
+  auto zero_w = [&]() {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = make_double2(0.0, 0.0);
-    with_count(live_q(m), [&](auto QC) {
-      constexpr int QN = decltype(QC)::value;
-      for (int i0 = 0; i0 < m; i0 += 4) {
-        cplx cli[4], dv[4][QN];
+    for (int e = 0; e < SB_TW; ++e)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          cli[t] = Cm[i0 + t][ga];
+      for (int q = 0; q < 4; ++q) wt[e][q] = make_double2(0.0, 0.0);
+  };
+  // f(e, row, column of register 0) for each of the wave's tiles that reaches into m x m
+  auto own_tiles = [&](auto&& f) {
 #pragma unroll
-          for (int q = 0; q < QN; ++q) dv[t][q] = Dm[i0 + t][gq + 8 * q];
-        }
+    for (int e = 0; e < SB_TW; ++e) {
+      const int t = wave + SB_W * e, l0 = 16 * (t % SB_M), j0 = 16 * (t / SB_M);
+      if (l0 < m && j0 < m) f(e, l0, j0);
+    }
+  };
+  auto w_to_lds = [&]() {
+    const int ln = here(lane), lr = ln & 15, lk = ln >> 4;
+    own_tiles([&](int e, int l0, int j0) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-#pragma unroll
-          for (int q = 0; q < QN; ++q) acc[q] = cfma(cli[t], dv[t][q], acc[q]);
-        }
+      for (int q = 0; q < 4; ++q) {
+        const int l = l0 + 4 * q + lk, j = j0 + lr;
+        if (l < SB_K && j < SB_K) Wm[l][j] = wt[e][q];
       }
     });
-#pragma unroll
-    for (int q = 0; q < 4; ++q) gs[1][ga + SB_K * (gq + 8 * q)] = acc[q];
   };
-  // Yhat(r, j) = delta(r, P_j) - G(P_j, r) into Y for j < m, rows of this thread
-  auto form_yhat = [&]() {
-    for (int r = tid; r < n; r += 256) {
+
+  zero_w();
+  int cur = 1, mb = 0;
+  bool cut = true;            // the records at vr[cur ^ 1] are not those of the visits from pos on
+  while (true) {
+    // ---- the end of the block before and the start of the next: its sites' rows and columns of
+    // G are in flight while W += Cn Dn^T over the m x m corner goes into the tiles and to LDS ----
+    const bool more = !stopped && pos < a.n_op && (m < kmax || a.final_round);
+    cplx gss[4], gsa[NE], gas[NE];
+    if (more) {
+      if (cut) {
+        if (wave == SB_W - 1) records(pos, cur ^ 1);
+        __syncthreads();
+      }
+      cur ^= 1;
+      gather(vr[cur], a.n_op - pos < SB_V ? a.n_op - pos : SB_V, gss, gsa, gas);
+    }
+    if (mb > 0) {
+      const int mb4 = (mb + 3) & ~3, ln = here(lane), lr = ln & 15, lk = ln >> 4;
+      own_tiles([&](int e, int l0, int j0) {
+        Tile3 c;
+        tile_mac(c, mb4, lk, [&](int i) { return Cn[i * SB_PL + l0 + lr]; },
+                 [&](int i) { return Dn[i * SB_PL + j0 + lr]; });
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (l0 + 4 * q + lk < m && j0 + lr < m) wt[e][q] = cadd(wt[e][q], c.get(q));
+      });
+    }
+    if (!more) break;
+    w_to_lds();
+    __syncthreads();   // the block's tables are free and W is complete
+    if (m >= kmax) {
+      // last round of the slice and the round is full: G += (G(:, A) W) Yhat^T in place
+      for (int r = tid; r < n; r += SB_T) {
+        for (int j = 0; j < m; ++j) {
+          const int P = s_aP[j];
+          const cplx g = a.G[P + (long long)r * n];
+          a.Y[r + (long long)j * n] = make_double2((r == P ? 1.0 : 0.0) - g.x, -g.y);
+          cplx acc = make_double2(0.0, 0.0);
+          for (int l = 0; l < m; ++l) acc = cfma(a.G[r + (long long)s_aP[l] * n], Wm[l][j], acc);
+          a.X[r + (long long)j * n] = acc;
+        }
+      }
+      __syncthreads();
+      for (int r = tid; r < n; r += SB_T) {
+        for (int c = 0; c < n; ++c) {
+          cplx acc = a.G[r + (long long)c * n];
+          for (int j = 0; j < m; ++j) acc = cfma(a.X[r + (long long)j * n], a.Y[c + (long long)j * n], acc);
+          a.G[r + (long long)c * n] = acc;
+        }
+      }
+      m = 0;
+      zero_w();
+      __syncthreads();
+      gather(vr[cur], a.n_op - pos < SB_V ? a.n_op - pos : SB_V, gss, gsa, gas);
+    }
+    const int nb = a.n_op - pos < SB_V ? a.n_op - pos : SB_V;
+    const int m4 = (m + 3) & ~3, mt = (m + 15) >> 4;
+    const BVisit* const vc = vr[cur];
+    if (m > 0) {
+      // ---- G[S, A] and Yhat[S, A] ----
+      const int ln = here(lane), lr = ln & 15, lk = ln >> 4, td = here(tid);
+      const int s = td & (SB_V - 1), Ps = vc[s < nb ? s : 0].P;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int l = (td >> 5) + (SB_T / SB_V) * e;
+        if (l < m) {
+          Xa[l][s] = make_double2(gsa[e].x, gsa[e].y);
+          Yh[l][s] = make_double2((Ps == s_aP[l] ? 1.0 : 0.0) - gas[e].x, -gas[e].y);
+        } else if (l < m4) {
+          Xa[l][s] = make_double2(0.0, 0.0);
+          Yh[l][s] = make_double2(0.0, 0.0);
+        }
+      }
+      __syncthreads();
+      // ---- T1 = G[S, A] W in place of G[S, A] (waves 0 .. 3), T2 = W Yhat[S, A]^T (4 .. 7):
+      //      tile t covers sites 16 (t % 2) and rows or columns 16 (t / 2) of W ----
+      constexpr int NT1 = (2 * SB_M + 3) / 4;
+      cplx t1[NT1][4];
+#pragma unroll
+      for (int q = 0; q < NT1; ++q) {
+        const int t = (wave & 3) + 4 * q;
+        if (t < 2 * mt) {
+          const int sc = 16 * (t & 1) + lr, j = 16 * (t >> 1) + lr;
+          const int jc = j < SB_K ? j : SB_K - 1;
+          Tile3 c;
+          if (wave < 4) {
+            tile_mac(c, m4, lk, [&](int k) { return Wm[k][jc]; }, [&](int k) { return Xa[k][sc]; });
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t1[q][r] = c.get(r);
+          } else {
+            tile_mac(c, m4, lk, [&](int k) { return Wm[jc][k]; }, [&](int k) { return Yh[k][sc]; });
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int l = 16 * (t >> 1) + 4 * r + lk;
+              if (l < SB_K) Wy[l][sc] = c.get(r);
+            }
+          }
+        }
+      }
+      __syncthreads();
+      if (wave < 4) {
+#pragma unroll
+        for (int q = 0; q < NT1; ++q) {
+          const int t = wave + 4 * q;
+          if (t < 2 * mt) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int j = 16 * (t >> 1) + 4 * r + lk;
+              if (j < SB_K) Xa[j][16 * (t & 1) + lr] = t1[q][r];
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+    // ---- g = G[S, S] + T1 Yhat[S, A]^T ----
+    if (wave < 4) {
+      const int ln = here(lane), lr = ln & 15, lk = ln >> 4;
+      const int r = 16 * (wave & 1) + lr, c0 = 16 * (wave >> 1);
+      Tile3 c;
+      tile_mac(c, m4, lk, [&](int k) { return Yh[k][c0 + lr]; }, [&](int k) { return Xa[k][r]; });
+#pragma unroll
+      for (int q = 0; q < 4; ++q) gs[c0 + 4 * q + lk][r] = cadd(gss[q], c.get(q));
+    } else {
+      // (T1 and T2 have read W, which lies below)
+      for (int e = here(tid) - 256; e < SB_A * 64; e += SB_T - 256) (&Tuw[0][0])[e] = make_double2(0.0, 0.0);
+      if (tid - 256 <= SB_A) s_pub[tid - 256] = 0;
+    }
+    __syncthreads();
+
+    // ---- the visits ----
+    // A rejected proposal leaves g and the phase unchanged, so the decisions of all visits up to
+    // the next acceptance follow from the same g: lane v (and v + 32) tests visit v, and the first
+    // passing visit at or after k is the next acceptance.  Each lane also forms what its visit
+    // would make of the phase and x = Delta / (1 + v_P Delta), v_P = 1 - G_cur(P,P), beside the test.
+    if (wave == 0) {
+      const int lane = here(tid), v = lane & (SB_V - 1);
+      const bool high = lane >= SB_V;
+      const BVisit rec = vc[v < nb ? v : nb - 1];
+      const int loc = rec.loc;
+      const unsigned have = (unsigned)__ballot(v < nb && rec.fnew != VISIT_NONE);
+      const int nvis = ~have == 0u ? SB_V : __builtin_ctz(~have);
+      // element p of this lane's row or column of g, and of the other half's u_i, w_i
+      const cplx* const g_lane = high ? &gs[v][0] : &gs[0][v];
+      const int g_step = high ? 1 : SB_PS;
+      const cplx* const t_lane = high ? &Tuw[0][0] : &Tuw[0][32];
+      cplx d = gs[v][v];
+      int k = nvis, mb = 0, js_of = 0;     // js_of: the visit of the block's flip number `lane`
+      unsigned live = nvis >= 32 ? ~0u : (1u << nvis) - 1u;
+      auto decide = [&](auto NS2) {
+        while (true) {
+          const cplx ratio = make_double2(fma(-rec.cb.x, d.x, fma(rec.cb.y, d.y, rec.ca.x)),
+                                          fma(-rec.cb.x, d.y, fma(-rec.cb.y, d.x, rec.ca.y)));
+          cplx rt = ratio;
+          if constexpr (decltype(NS2)::value) rt = cmul(ratio, ratio);
+          else for (int s = 1; s < a.n_sun; ++s) rt = cmul(rt, ratio);
+          const cplx zn = cmul(z, rt);
+          const bool pass = fabs(zn.x) > rec.thr * fabs(z.x);
+          const cplx delta = rec.delta;
+          const cplx den = make_double2(1.0 + (1.0 - d.x) * delta.x + d.y * delta.y,
+                                        (1.0 - d.x) * delta.y - d.y * delta.x);
+          const double c2 = cabs2(den);
+          double rden = __builtin_amdgcn_rcp(c2);          // two Newton steps: full precision
+          rden = fma(fma(-c2, rden, 1.0), rden, rden);
+          rden = fma(fma(-c2, rden, 1.0), rden, rden);
+          const cplx xl = cscale(cmul(delta, cconj(den)), rden);
+          // keep these beside the test, where its latency leaves room, instead of after the ballot
+          __asm__ volatile("" ::"v"(xl.x), "v"(xl.y), "v"(zn.x), "v"(zn.y));
+          const unsigned lo = (unsigned)__ballot(pass) & live;   // lanes 0..31: visits 0..31 of the block
+          if (lo == 0) return;
+          const int js = __builtin_amdgcn_readfirstlane(__builtin_ctz(lo));
+          const int p = __builtin_amdgcn_readlane(loc, js);
+          live &= ~1u << js;
+          // column p (low lanes) and row p (high lanes) of the current g
+          cplx col = g_lane[p * g_step], sum = make_double2(0.0, 0.0);
+          const cplx* const oth = t_lane + p;
+          // this lane's u_{mb} (low) = -x col, w_{mb} (high) = delta - col, as f0 + f1 col
+          cplx f1;
+          double f0;
+          auto dot = [&](auto C) {
+            constexpr int IN = decltype(C)::value;
+            cplx mine[IN], their[IN];
+#pragma unroll
+            for (int i = 0; i < IN; ++i) {
+              mine[i] = Tuw[i][lane];
+              their[i] = oth[64 * i];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // in the shadow of the reads
+            const cplx x = lane_c(xl, js);
+            f0 = high && loc == p ? 1.0 : 0.0;
+            f1 = high ? make_double2(-1.0, 0.0) : make_double2(-x.x, -x.y);
+            z = lane_c(a.n_sun <= 4 ? zn : renorm_pow2(zn), js);
+            js_of = lane == mb ? js : js_of;
+#pragma unroll
+            for (int i = 0; i < IN; i += 2) {
+              col = cfma(mine[i], their[i], col);
+              sum = cfma(mine[i + 1], their[i + 1], sum);
+            }
+          };
+          // (u_i, w_i are zero for the flips not yet made)
+          if (mb <= 4) dot(std::integral_constant<int, 4>{});
+          else if (mb <= 8) dot(std::integral_constant<int, 8>{});
+          else {
+            dot(std::integral_constant<int, 8>{});
+            for (int i0 = 8; i0 < mb; i0 += 4) {
+              cplx mine[4], their[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                mine[i] = Tuw[i0 + i][lane];
+                their[i] = oth[64 * (i0 + i)];
+              }
+#pragma unroll
+              for (int i = 0; i < 4; i += 2) {
+                col = cfma(mine[i], their[i], col);
+                sum = cfma(mine[i + 1], their[i + 1], sum);
+              }
+            }
+          }
+          col = cadd(col, sum);
+          const cplx res = make_double2(fma(f1.x, col.x, fma(-f1.y, col.y, f0)), fma(f1.x, col.y, f1.y * col.x));
+          Tuw[mb][lane] = res;
+          // g(v, v) += u(v) w(v)
+          double ux, uy, wx, wy;
+          both_halves(res.x, ux, wx);
+          both_halves(res.y, uy, wy);
+          d = cfma(make_double2(ux, uy), make_double2(wx, wy), d);
+          if (lane == js) {
+            s_x[mb] = xl;
+            publish(mb, p + 1);
+          }
+          mb = __builtin_amdgcn_readfirstlane(mb + 1);
+          if (m + mb >= kmax || mb >= SB_A) {
+            k = js + 1;
+            return;
+          }
+        }
+      };
+      if (a.n_sun == 2) decide(std::true_type{});
+      else decide(std::false_type{});
+      z = renorm_pow2(z);
+      if (lane < mb) {
+        const BVisit& w = vc[js_of];
+        a.f[(long long)a.slice * a.n_op + (a.dir > 0 ? pos + js_of : a.n_op - 1 - pos - js_of)] = (int8_t)w.fnew;
+        s_aP[m + lane] = w.P;
+      }
+      if (lane == 0) {
+        s_mb = mb;
+        s_k = k;
+        s_stopped = k == nvis && nvis < nb;   // the random stream ends here
+        publish(mb, SB_FIN);
+      }
+    } else if (wave <= 2) {
+      // ---- columns Cn (wave 1) and Dn (wave 2), row l of W in lane l ----
+      const bool isc = wave == 1;
+      const int l = here(lane), lc = l < SB_K ? l : SB_K - 1;
+      const cplx* const T = isc ? &Wy[lc][0] : &Xa[lc][0];   // T2(l, :) / T1(:, l)
+      const cplx* const N = &Tuw[0][isc ? 32 : 0];           // w_i(p) / u_i(p)
+      cplx* const out = isc ? Cn : Dn;
+      int j = 0;
+      while (true) {
+        const int pub = __hip_atomic_load(&s_pub[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        lds_order();
+        if (pub == 0) {
+          __builtin_amdgcn_s_sleep(1);
+          continue;
+        }
+        if (pub == SB_FIN) break;             // the deciding wave always ends with SB_FIN
+        const int p = pub - 1;
+        const cplx x = s_x[j];
+        cplx acc = l < m ? T[p] : make_double2(0.0, 0.0), acc1 = make_double2(0.0, 0.0);
+        for (int i0 = 0; i0 < j; i0 += 4) {
+          cplx mine[4], their[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int ii = i0 + i < j ? i0 + i : 0;
+            mine[i] = l < SB_K ? out[ii * SB_PL + l] : make_double2(0.0, 0.0);
+            their[i] = i0 + i < j ? N[64 * ii + p] : make_double2(0.0, 0.0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i += 2) {
+            acc = cfma(mine[i], their[i], acc);
+            acc1 = cfma(mine[i + 1], their[i + 1], acc1);
+          }
+        }
+        acc = cadd(acc, acc1);
+        const double dl = l == m + j ? 1.0 : 0.0;
+        const cplx r = isc ? cmul(make_double2(-x.x, -x.y), make_double2(dl + acc.x, acc.y))
+                           : make_double2(dl - acc.x, -acc.y);
+        if (l < SB_K) out[j * SB_PL + l] = r;
+        ++j;
+      }
+      // zero up to a whole k-step of the product below
+      for (; j & 3; ++j)
+        if (l < SB_K) out[j * SB_PL + l] = make_double2(0.0, 0.0);
+    } else if (wave == SB_W - 1) {
+      // the records of the block after this one, if this one is not cut short
+      records(pos + nb, cur ^ 1);
+    }
+    __syncthreads();
+    mb = s_mb;
+    const int k = s_k;
+    stopped = s_stopped != 0;
+    m += mb;
+    nvisits += k;
+    naccepts += mb;
+    cut = k < nb;                            // the next block does not start where the records do
+    pos += k;
+  }
+  // ---- the round's flush operands: W (zero up to whole tiles of 16), the site list, Yhat ----
+  own_tiles([&](int e, int l0, int j0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a.W[l0 + 4 * q + lk + CHAIN_W_LD * (j0 + lr)] = wt[e][q];
+  });
+  if (!a.yhat_external) {
+    // Yhat(r, j) = delta(r, P_j) - G(P_j, r)
+    for (int r = tid; r < n; r += SB_T) {
       for (int j0 = 0; j0 < m; j0 += 8) {
         cplx gv[8];
 #pragma unroll
@@ -423,320 +842,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             a.Y[r + (long long)(j0 + t) * n] = make_double2((r == s_aP[j0 + t] ? 1.0 : 0.0) - gv[t].x, -gv[t].y);
       }
     }
-  };
-
-  zero_cd();
-  while (pos < a.n_op) {
-    if (m >= kmax) {
-      if (!a.final_round) break;
-      // last round of the slice and the round is full: G += (G(:, A) W) Yhat^T in place
-      form_w();
-      form_yhat();
-      __syncthreads();
-      for (int r = tid; r < n; r += 256) {
-        for (int j = 0; j < m; ++j) {
-          cplx acc = make_double2(0.0, 0.0);
-          for (int l = 0; l < m; ++l) acc = cfma(a.G[r + (long long)s_aP[l] * n], gs[1][l + SB_K * j], acc);
-          a.X[r + (long long)j * n] = acc;
-        }
-      }
-      __syncthreads();
-      for (int r = tid; r < n; r += 256) {
-        for (int c = 0; c < n; ++c) {
-          cplx acc = a.G[r + (long long)c * n];
-          for (int j = 0; j < m; ++j) acc = cfma(a.X[r + (long long)j * n], a.Y[c + (long long)j * n], acc);
-          a.G[r + (long long)c * n] = acc;
-        }
-      }
-      m = 0;
-      zero_cd();
-      __syncthreads();
-    }
-    int nb = a.n_op - pos < SB_V ? a.n_op - pos : SB_V;
-    if (!have_records || pos + nb > vbase + SB_R) {
-      vbase = pos;
-      build_records();
-    }
-    const int r0 = pos - vbase;
-    int nvis = stop_at - pos < nb ? stop_at - pos : nb;
-    if (nvis < 0) nvis = 0;
-    // ---- block start: the sites' indices in the block (wave 0), G at the block's sites,
-    //      G[S, A] and Yhat[S, A] for the round's earlier flips ----
-    if (tid < SB_V) {
-      const int Pw = vr[r0 + (tid < nb ? tid : 0)].P;
-      int loc = tid;
-      for (int t = 0; t < SB_V; ++t) {
-        const int Pt = __builtin_amdgcn_readlane(Pw, t);
-        if (t < tid && t < nb && tid < nb && Pt == Pw && loc == tid) loc = t;
-      }
-      if (tid < nb) vr[r0 + tid].loc = loc;
-    }
-    cplx gown[4];
-    {
-      const int Pa = vr[r0 + (ga < nb ? ga : 0)].P;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = gq + 8 * q;
-        const cplx gv = a.G[Pa + (long long)vr[r0 + (b < nb ? b : 0)].P * n];
-        gown[q] = (ga < nb && b < nb) ? gv : make_double2(0.0, 0.0);
-      }
-    }
-    {
-      const int s = ga, Ps = vr[r0 + (s < nb ? s : 0)].P;
-      cplx gsa[4], gas[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int l = gq + 8 * q;
-        const int Pl = l < m ? s_aP[l] : 0;
-        gsa[q] = a.G[Ps + (long long)Pl * n];
-        gas[q] = a.G[Pl + (long long)Ps * n];
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int l = gq + 8 * q;
-        const bool live = s < nb && l < m;
-        const int Pl = l < m ? s_aP[l] : 0;
-        gs[1][s + SB_V * l] = live ? gsa[q] : make_double2(0.0, 0.0);
-        UW[s + SB_V * l] = live ? make_double2((Ps == Pl ? 1.0 : 0.0) - gas[q].x, -gas[q].y) : make_double2(0.0, 0.0);
-      }
-    }
-    __syncthreads();
-    // X[S, j] = sum_l G[S, A_l] C(l, j),  Y[S, j] = sum_l Yhat[S, A_l] D(l, j)   (zero for j >= m)
-    {
-      cplx ax[4], ay[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) { ax[q] = make_double2(0.0, 0.0); ay[q] = make_double2(0.0, 0.0); }
-      with_count(live_q(m), [&](auto QC) {
-        constexpr int QN = decltype(QC)::value;
-        for (int l0 = 0; l0 < m; l0 += 4) {
-          cplx gl[4], yl[4], cv[4][QN], dv[4][QN];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            gl[t] = gs[1][ga + SB_V * (l0 + t)];
-            yl[t] = UW[ga + SB_V * (l0 + t)];
-#pragma unroll
-            for (int q = 0; q < QN; ++q) {
-              cv[t][q] = Cm[gq + 8 * q][l0 + t];
-              dv[t][q] = Dm[gq + 8 * q][l0 + t];
-            }
-          }
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-#pragma unroll
-            for (int q = 0; q < QN; ++q) {
-              ax[q] = cfma(gl[t], cv[t][q], ax[q]);
-              ay[q] = cfma(yl[t], dv[t][q], ay[q]);
-            }
-          }
-        }
-      });
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        Xb[gq + 8 * q][ga] = ax[q];
-        Yb[gq + 8 * q][ga] = ay[q];
-      }
-    }
-    __syncthreads();
-    for (int i0 = 0; i0 < m; i0 += 4) {
-      cplx xa[4], yv[4][4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        xa[t] = Xb[i0 + t][ga];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) yv[t][q] = Yb[i0 + t][gq + 8 * q];
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) gown[q] = cfma(xa[t], yv[t][q], gown[q]);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) gs[0][ga + SB_V * (gq + 8 * q)] = gown[q];
-    __syncthreads();
-
-    // ---- the visits: decisions from g, rank-1 updates of g on acceptance ----
-    // A rejected proposal leaves g and the phase unchanged, so the decisions of all visits
-    // up to the next acceptance follow from the same g: lane j (= ga) decides visit j of
-    // the block with the record and diagonal entry of that visit, and the first visit at
-    // or after k whose test passes is the next acceptance (every one before it is
-    // rejected).  Each lane also forms its visit's x = Delta / (1 + v_P Delta), so the
-    // division runs beside the test.  The arithmetic of each decision is that of a
-    // sequential visit with the same g(p, p) and phase.
-    int buf = 0, mb = 0, k = 0;
-    const BVisit rec = vr[r0 + (ga < nb ? ga : nb - 1)];
-    const int2 rec_aux = vaux[r0 + (ga < nb ? ga : nb - 1)];
-    const bool lane_live = ga < nvis;
-    while (k < nvis) {
-      const cplx d = gs[buf][rec.loc * (SB_V + 1)];
-      const cplx ratio = make_double2(fma(-rec.cb.x, d.x, fma(rec.cb.y, d.y, rec.ca.x)),
-                                      fma(-rec.cb.x, d.y, fma(-rec.cb.y, d.x, rec.ca.y)));
-      cplx rt = ratio;
-      if (a.n_sun == 2) rt = cmul(ratio, ratio);
-      else for (int s = 1; s < a.n_sun; ++s) rt = cmul(rt, ratio);
-      const double lhs = fabs(fma(z.x, rt.x, -z.y * rt.y));
-      // x = Delta / (1 + v_P Delta), v_P = 1 - G_cur(P,P)
-      const cplx delta = rec.delta;
-      const cplx den = make_double2(1.0 + (1.0 - d.x) * delta.x + d.y * delta.y,
-                                    (1.0 - d.x) * delta.y - d.y * delta.x);
-      const double rden = 1.0 / cabs2(den);
-      const cplx xl = cscale(cmul(delta, cconj(den)), rden);
-      // keep the division here, beside the test, instead of after the ballot
-      __asm__ volatile("" ::"v"(xl.x), "v"(xl.y));
-      const bool pass = lane_live && ga >= k && lhs > rec.thr * fabs(z.x);
-      const unsigned lo = (unsigned)__ballot(pass);   // lanes 0..31: visits 0..31 of the block
-      if (lo == 0) {
-        k = nvis;
-        break;
-      }
-      const int js = __builtin_amdgcn_readfirstlane(__builtin_ctz(lo));
-      k = js + 1;
-      z = renorm_pow2(cmul(z, lane_c(rt, js)));
-      const cplx x = lane_c(xl, js);
-      const int p = __builtin_amdgcn_readlane(rec.loc, js);
-      const int P_acc = __builtin_amdgcn_readlane(rec.P, js);
-      const int f_new = __builtin_amdgcn_readlane(rec_aux.x, js), op_acc = __builtin_amdgcn_readlane(rec_aux.y, js);
-      const cplx mx = make_double2(-x.x, -x.y);
-      const cplx gcol = gs[buf][ga + SB_V * p];
-      cplx gpb[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) gpb[q] = gs[buf][p + SB_V * (gq + 8 * q)];
-      const cplx ua = cmul(mx, gcol);
-      cplx wb[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = gq + 8 * q;
-        wb[q] = make_double2((b == p ? 1.0 : 0.0) - gpb[q].x, -gpb[q].y);
-        gown[q] = cfma(ua, wb[q], gown[q]);
-        gs[buf ^ 1][ga + SB_V * b] = gown[q];
-      }
-      if (gq == 0) Us[mb * SB_V + ga] = ua;
-      if (ga == 0) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) Ws[mb * SB_V + gq + 8 * q] = wb[q];
-        if (tid == 0) {
-          a.f[(long long)a.slice * a.n_op + op_acc] = (int8_t)f_new;
-          s_x[m + mb] = x;
-          s_aP[m + mb] = P_acc;
-          s_aloc[mb] = p;
-        }
-      }
-      mb += 1;
-      buf ^= 1;
-      block_sync_lds();
-      if (m + mb >= kmax || mb >= SB_A) break;
-    }
-    nvisits += k;
-    naccepts += mb;
-    pos += k;
-    if (k == nvis && pos == stop_at && stop_at < a.n_op) stopped = true;   // random stream exhausted here
-
-    // ---- extend C and D by the block's flips ----
-    if (mb > 0) {
-      __syncthreads();   // every wave is past its last visit (gs[1] is reused below)
-      // (1) the part over the round's earlier flips, for every (row l, new column jj):
-      //     pre(l, jj) = sum_{i < m} M(l, i) L(i, p_jj), L = Y(P, i) for C and X(P, i) for D;
-      //     threads: matrix (tid / 128), row l, four columns jj = c4 + 4 t each
-      cplx* const Pre = gs[1];   // [matrix][jj][l]
-      {
-        const int mat = tid >> 7, l = (tid >> 2) & (SB_K - 1), c4 = tid & 3;
-        cplx(*Mm)[SB_K] = mat ? Dm : Cm;
-        cplx(*Lold)[SB_V] = mat ? Xb : Yb;
-        // columns jj < 4 TN, TN = ceil(mb / 4), cover the block's flips
-        with_count(__builtin_amdgcn_readfirstlane((mb + 3) >> 2), [&](auto TC) {
-          constexpr int TN = decltype(TC)::value;
-          cplx acc[TN];
-          int pj[TN];
-#pragma unroll
-          for (int t = 0; t < TN; ++t) {
-            acc[t] = make_double2(0.0, 0.0);
-            const int jj = c4 + 4 * t;
-            pj[t] = s_aloc[jj < mb ? jj : 0];
-          }
-          for (int i0 = 0; i0 < m; i0 += 4) {
-            cplx mli[4], lv[4][TN];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              mli[u] = Mm[i0 + u][l];
-#pragma unroll
-              for (int t = 0; t < TN; ++t) lv[u][t] = Lold[i0 + u][pj[t]];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-#pragma unroll
-              for (int t = 0; t < TN; ++t) acc[t] = cfma(mli[u], lv[u][t], acc[t]);
-            }
-          }
-#pragma unroll
-          for (int t = 0; t < TN; ++t) Pre[(mat * SB_A + c4 + 4 * t) * SB_K + l] = acc[t];
-        });
-      }
-      __syncthreads();
-      // (2) the in-block recurrence, one thread per (matrix, row), new entries in registers.
-      //     Right-looking: once entry jj is final its terms go into the sums of every later
-      //     column, and each table entry of row jj, once used, is replaced by the same column's
-      //     entry of row jj + 1, so the next row's reads are in flight while this row's terms
-      //     are added.  Each sum still adds its terms in the order ii = 0, 1, ...  Columns up to
-      //     4 ceil(mb / 4) are carried without branches; those at or beyond mb are not stored.
-      if (tid < 2 * SB_K) {
-        const int mat = tid >> 5, l = tid & (SB_K - 1);
-        const cplx* Lnew = mat ? Us : Ws;   // X(P_j, i) = u_i(p_j) / Y(P_j, i) = w_i(p_j)
-        cplx(*Mm)[SB_K] = mat ? Dm : Cm;
-        with_count(__builtin_amdgcn_readfirstlane((mb + 3) >> 2), [&](auto TC) {
-          constexpr int JN = 4 * decltype(TC)::value;
-          cplx acc[JN], lr[JN];
-          int pj[JN];
-#pragma unroll
-          for (int jj = 0; jj < JN; ++jj) {
-            pj[jj] = s_aloc[jj < mb ? jj : 0];
-            acc[jj] = Pre[(mat * SB_A + jj) * SB_K + l];
-          }
-#pragma unroll
-          for (int kk = 1; kk < JN; ++kk) lr[kk] = Lnew[pj[kk]];
-#pragma unroll
-          for (int jj = 0; jj < JN; ++jj) {
-            const int j = m + jj;
-            const cplx xj = s_x[j < SB_K ? j : SB_K - 1];
-            const double dl = l == j ? 1.0 : 0.0;
-            const cplx vd = make_double2(dl - acc[jj].x, -acc[jj].y);
-            const cplx vc = cmul(make_double2(-xj.x, -xj.y), make_double2(dl + acc[jj].x, acc[jj].y));
-            const cplx v = (jj < mb && l <= j) ? (mat ? vd : vc) : make_double2(0.0, 0.0);
-            if (jj < mb) Mm[j][l] = v;
-#pragma unroll
-            for (int kk = jj + 1; kk < JN; ++kk) {
-              acc[kk] = cfma(v, lr[kk], acc[kk]);
-              if (kk > jj + 1) lr[kk] = Lnew[(jj + 1) * SB_V + pj[kk]];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        });
-      }
-      m += mb;
-    }
-    __syncthreads();   // the LDS tables of the block are free, C and D are complete
-    if (stopped) break;
   }
-  // ---- the round's flush operands: W = C D^T, the site list, Yhat ----
-  form_w();
-  if (!a.yhat_external) form_yhat();
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 4; ++q) a.W[ga + SB_K * (gq + 8 * q)] = gs[1][ga + SB_K * (gq + 8 * q)];
-  if (tid < SB_K) a.amap[tid] = tid < m ? s_aP[tid] : 0;
+  if (tid < CHAIN_KMAX) a.amap[tid] = tid < m ? s_aP[tid] : 0;
   if (tid == 0) {
     st->phase = cscale(z, 1.0 / sqrt(cabs2(z)));
-    st->nc = s_nc + nvisits;
-    st->acc = s_accn + naccepts;
-    st->pos = pos;
+    st->nc = st0.nc + nvisits;
+    st->acc = st0.acc + naccepts;
     st->m = m;
-    st->rng_slice_base = base;
-    st->rng_pos = base + (unsigned long long)a.uoff[pos];
-    st->slice_acc += (int)naccepts;
+    const int sl = st0.slice_acc + (int)naccepts;
+    st->slice_acc = sl;
     if (stopped) {
       st->status = 1;
-      st->pos = a.n_op;    // do not revisit
+      st->rng_pos = st0.rng_pos + (unsigned long long)a.uoff[pos];
     }
-    if (st->pos >= a.n_op && st->slice_acc > st->max_slice_acc) st->max_slice_acc = st->slice_acc;
+    if (stopped || pos >= a.n_op) {
+      // the slice is done (a stopped one is not revisited) and the stream behind it
+      if (!stopped) st->rng_pos = st0.rng_pos + (unsigned long long)a.per;
+      if (sl > st0.max_slice_acc) st->max_slice_acc = sl;
+      pos = a.n_op;
+    }
+    st->pos = pos;
   }
 }
 
@@ -809,6 +934,14 @@ int launch_philox_fill(double* u, ChainState* st, long long count, int nchain, l
   return ST_NONE;
 }
 
+int launch_visits(const VisitArgs& a, hipStream_t s) {
+  const long long count = (long long)a.n_op * a.ns;
+  if (count <= 0) return ST_NONE;
+  hipLaunchKernelGGL(visit_kernel, dim3((unsigned)((count + 255) / 256), 1, a.nchain), dim3(256), 0, s, a);
+  HIP_OK(hipGetLastError());
+  return ST_NONE;
+}
+
 int chain_max_delay(int n) {
   (void)n;
   return SB_K;
@@ -819,7 +952,7 @@ int launch_chain(const ChainArgs& a, hipStream_t s, KTimer* t) {
     alfq_set_error("launch_chain: K outside [1, CHAIN_KMAX]");
     return ST_GENERIC;
   }
-  if (a.Kmax <= SB_K && a.uoff) {
+  if (a.Kmax <= SB_K && a.rec) {
     if (t && t->on) {
       if (t->used == t->ev.size()) {
         hipEvent_t e0, e1;
@@ -830,9 +963,9 @@ int launch_chain(const ChainArgs& a, hipStream_t s, KTimer* t) {
         t->ev.emplace_back(e0, e1);
       }
       auto& pr = t->ev[t->used++];
-      hipExtLaunchKernelGGL(chain_block_kernel, dim3(1, 1, a.nchain), dim3(256), 0, s, pr.first, pr.second, 0, a);
+      hipExtLaunchKernelGGL(chain_block_kernel, dim3(1, 1, a.nchain), dim3(SB_T), 0, s, pr.first, pr.second, 0, a);
     } else {
-      hipLaunchKernelGGL(chain_block_kernel, dim3(1, 1, a.nchain), dim3(256), 0, s, a);
+      hipLaunchKernelGGL(chain_block_kernel, dim3(1, 1, a.nchain), dim3(SB_T), 0, s, a);
     }
     HIP_OK(hipGetLastError());
     return ST_NONE;

@@ -18,6 +18,7 @@
 //   * UDV chain      U <- D exp(-dtau T) U,  U <- exp(-dtau T) conj(D) U
 //   * delayed-update flush  G += X Y^T
 //   * QR trailing updates / Q formation / TRMM / CGR products
+#include "alfq_chain.h"
 #include "alfq_common.h"
 
 namespace {
@@ -599,16 +600,17 @@ __global__ __launch_bounds__(NT, 2) void gemm_tile_kernel(GemmArgs g) {
   }
 }
 
-// Delayed-update flush G += X Y^T of rank m <= 32 (the block kernel's round).  A workgroup
-// owns a 64 x 64 tile of one chain's G; its operands (the m columns of X for the tile's rows
-// and of Y for its columns) and the tile of G itself, read directly in the MFMA result
-// layout, are all requested at the start, so a tile costs one memory round trip; the
-// product takes ceil(m / 4) k-steps of 2 x 2 MFMA blocks per wave and G is written once.
-constexpr int FL_T = 64, FL_K = 32;
+// Delayed-update flush G += X Y^T of rank m <= CHAIN_BLOCK_KMAX (the block kernel's round).  A
+// workgroup owns a 64 x 64 tile of one chain's G; the tile itself, in the layout of the product,
+// and the first 16 columns of X (for the tile's rows) and Y (for its columns) are requested at
+// the start, the next 16 columns while the ones before them are multiplied, and G is written once.
+// Bound by the traffic of G (2 x 16 n^2 bytes per chain) and, from m ~ 45 on, by the FP64 matrix
+// rate; X Y^T is three real products (3M).
+constexpr int FL_T = 64, FL_C = 16;
 __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, const cplx* Y, const int* mdev,
                                                       int n, int kmax, long long cs) {
   typedef Mma<false> M;
-  __shared__ double Xr[FL_K][FL_T + 1], Xi[FL_K][FL_T + 1], Yr[FL_K][FL_T + 1], Yi[FL_K][FL_T + 1];
+  __shared__ cplx Xs[2][FL_C][FL_T + 1], Ys[2][FL_C][FL_T + 1];
   int bx, by, bz;
   xcd_order(bx, by, bz);
   G = chain_ptr_at(G, cs, bz);
@@ -623,16 +625,18 @@ __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, co
   const int wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
   const int wr = 32 * (wave & 1), wc = 32 * (wave >> 1);
   const int li = tid & 63, lkb = tid >> 6;   // operand rows: index li, columns k = lkb + 4 p
+  const int xi = i0 + li < n ? i0 + li : n - 1, yi = j0 + li < n ? j0 + li : n - 1;
 
-  cplx xv[FL_K / 4], yv[FL_K / 4];
+  cplx xv[FL_C / 4], yv[FL_C / 4];
+  auto load = [&](int k0) {
 #pragma unroll
-  for (int p = 0; p < FL_K / 4; ++p) {
-    const int k = lkb + 4 * p;
-    xv[p] = make_double2(0.0, 0.0);
-    yv[p] = make_double2(0.0, 0.0);
-    if (k < m && i0 + li < n) xv[p] = X[i0 + li + (long long)k * n];
-    if (k < m && j0 + li < n) yv[p] = Y[j0 + li + (long long)k * n];
-  }
+    for (int p = 0; p < FL_C / 4; ++p) {
+      const int k = k0 + lkb + 4 * p < m ? k0 + lkb + 4 * p : m - 1;
+      xv[p] = X[xi + (long long)k * n];
+      yv[p] = Y[yi + (long long)k * n];
+    }
+  };
+  load(0);
   cplx gv[2][2][4];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -640,51 +644,41 @@ __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, co
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gi = i0 + wr + 16 * a + M::row(r, lk), gj = j0 + wc + 16 * b + lr;
+        const int gi = i0 + wr + 16 * a + lr, gj = j0 + wc + 16 * b + M::row(r, lk);
         gv[a][b][r] = make_double2(0.0, 0.0);
         if (gi < n && gj < n) gv[a][b][r] = G[gi + (long long)gj * n];
       }
-#pragma unroll
-  for (int p = 0; p < FL_K / 4; ++p) {
-    const int k = lkb + 4 * p;
-    Xr[k][li] = xv[p].x;
-    Xi[k][li] = xv[p].y;
-    Yr[k][li] = yv[p].x;
-    Yi[k][li] = yv[p].y;
-  }
-  __syncthreads();
-
-  v4d acc_re[2][2], acc_im[2][2];
+  v4d acc_re[2][2], acc_im[2][2], acc_t2[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      acc_re[a][b] = v4d{0, 0, 0, 0};
-      acc_im[a][b] = v4d{0, 0, 0, 0};
+    for (int b = 0; b < 2; ++b) acc_re[a][b] = acc_im[a][b] = acc_t2[a][b] = v4d{0, 0, 0, 0};
+  int buf = 0;
+  for (int k0 = 0; k0 < m; k0 += FL_C, buf ^= 1) {
+#pragma unroll
+    for (int p = 0; p < FL_C / 4; ++p) {
+      const bool live = k0 + lkb + 4 * p < m;
+      Xs[buf][lkb + 4 * p][li] = live ? xv[p] : make_double2(0.0, 0.0);
+      Ys[buf][lkb + 4 * p][li] = live ? yv[p] : make_double2(0.0, 0.0);
     }
-  for (int k0 = 0; k0 < m; k0 += 4) {
-    const int kk = k0 + lk;
-    double a_re[2], a_im[2], b_re[2], b_im[2];
+    __syncthreads();
+    if (k0 + FL_C < m) load(k0 + FL_C);
+    const int kn = m - k0 < FL_C ? m - k0 : FL_C;
+    for (int kq = 0; kq < kn; kq += 4) {
+      cplx fa[2], fb[2];
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      a_re[a] = Xr[kk][wr + 16 * a + lr];
-      a_im[a] = Xi[kk][wr + 16 * a + lr];
-    }
+      for (int a = 0; a < 2; ++a) fa[a] = Xs[buf][kq + lk][wr + 16 * a + lr];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      b_re[b] = Yr[kk][wc + 16 * b + lr];
-      b_im[b] = Yi[kk][wc + 16 * b + lr];
-    }
+      for (int b = 0; b < 2; ++b) fb[b] = Ys[buf][kq + lk][wc + 16 * b + lr];
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const double na = -a_im[a];
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        acc_re[a][b] = M::mac(a_re[a], b_re[b], acc_re[a][b]);
-        acc_im[a][b] = M::mac(a_re[a], b_im[b], acc_im[a][b]);
-        acc_re[a][b] = M::mac(na, b_im[b], acc_re[a][b]);
-        acc_im[a][b] = M::mac(a_im[a], b_re[b], acc_im[a][b]);
-      }
+        for (int b = 0; b < 2; ++b) {
+          // operands exchanged: the 16 lanes of a result row run along a column of G
+          acc_re[a][b] = M::mac(fb[b].x, fa[a].x, acc_re[a][b]);
+          acc_t2[a][b] = M::mac(fb[b].y, fa[a].y, acc_t2[a][b]);
+          acc_im[a][b] = M::mac(fb[b].x + fb[b].y, fa[a].x + fa[a].y, acc_im[a][b]);
+        }
     }
   }
 #pragma unroll
@@ -693,9 +687,11 @@ __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, co
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gi = i0 + wr + 16 * a + M::row(r, lk), gj = j0 + wc + 16 * b + lr;
+        const int gi = i0 + wr + 16 * a + lr, gj = j0 + wc + 16 * b + M::row(r, lk);
+        const double re = acc_re[a][b][r], t2 = acc_t2[a][b][r];
         if (gi < n && gj < n)
-          G[gi + (long long)gj * n] = make_double2(gv[a][b][r].x + acc_re[a][b][r], gv[a][b][r].y + acc_im[a][b][r]);
+          G[gi + (long long)gj * n] =
+              make_double2(gv[a][b][r].x + (re - t2), gv[a][b][r].y + (acc_im[a][b][r] - re - t2));
       }
 }
 
@@ -939,19 +935,21 @@ void launch_direct(const GemmArgs& g, hipStream_t s) {
 
 // The end of a delayed-update round for a few chains, in one launch:
 //   Go = Gi + (Gi(:, A) W) Yhat^T,   Yhat(c, j) = delta(c, P_j) - Gi(P_j, c),
-// A = (P_0 .. P_{m-1}) the round's accepted sites, W = C D^T (m x m, ld FL_K), m = *mdev.
-// Gi is only read and Go only written (two buffers), so a workgroup can gather the columns A
-// and rows A of Gi that it needs while others write their tiles.  A workgroup of two waves
-// owns a 16 x 16 tile: wave w forms columns 16w .. 16w + 15 of its rows of X = Gi(:, A) W,
-// then the waves split the rank-m product over k and add their halves through LDS.  Every
-// global load of the tile is issued before the first MFMA.
-constexpr int RF_T = 16;
-__global__ __launch_bounds__(128, 2) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
-                                                          const cplx* __restrict__ W, const int* __restrict__ amap,
-                                                          const int* mdev, int n, int kmax, long long cs) {
+// A = (P_0 .. P_{m-1}) the round's accepted sites, W m x m with leading dimension CHAIN_W_LD,
+// m = *mdev <= CHAIN_BLOCK_KMAX.  Gi is only read and Go only written (two buffers), so a
+// workgroup can gather the columns A and rows A of Gi that it needs while others write their
+// tiles.  A workgroup of RF_W waves owns a 16 x 16 tile: wave w forms columns 16 w .. 16 w + 15 of
+// its rows of X = Gi(:, A) W, then takes the same 16 of the rank-m product, and the parts are
+// added through LDS.  Latency-bound: every global load of the tile is issued before the first MFMA,
+// and the sites are read beside m so that the gathers wait for one load.
+constexpr int RF_T = 16, RF_W = (CHAIN_BLOCK_KMAX + 15) / 16, RF_K = 16 * RF_W;
+__global__ __launch_bounds__(64 * RF_W, 2) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
+                                                                  const cplx* __restrict__ W,
+                                                                  const int* __restrict__ amap, const int* mdev,
+                                                                  int n, int kmax, long long cs) {
   typedef Mma<false> M;
-  __shared__ cplx Xs[RF_T][FL_K + 1];
-  __shared__ cplx red[RF_T * RF_T];
+  __shared__ cplx Xs[RF_T][RF_K + 1];
+  __shared__ cplx red[RF_W - 1][RF_T * RF_T];
   const int z = blockIdx.z;
   Gi = chain_ptr_at(Gi, cs, z);
   Go = chain_ptr_at(Go, cs, z);
@@ -963,40 +961,37 @@ __global__ __launch_bounds__(128, 2) void round_flush_kernel(const cplx* __restr
   const int i0 = blockIdx.x * RF_T, j0 = blockIdx.y * RF_T;
   const int gi = i0 + lr, gj = j0 + lr;
   const bool row_ok = gi < n, col_ok = gj < n;
-  // the rank m and the sites are loaded together (the sites' buffer holds at least kmax
-  // entries), so the gathers below wait for one load instead of two
-  int pa[FL_K / 4], py[4];
+  // (the sites' buffer holds CHAIN_KMAX >= RF_K entries)
+  int pa[RF_K / 4], py[4];
 #pragma unroll
-  for (int u = 0; u < FL_K / 4; ++u) pa[u] = 4 * u + lk < kmax ? amap[4 * u + lk] : 0;
+  for (int u = 0; u < RF_K / 4; ++u) pa[u] = amap[4 * u + lk];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) py[u] = 16 * wave + 4 * u + lk < kmax ? amap[16 * wave + 4 * u + lk] : 0;
+  for (int u = 0; u < 4; ++u) py[u] = amap[16 * wave + 4 * u + lk];
   int m = *mdev;
   m = m < kmax ? m : kmax;
   m = m > 0 ? m : 0;
+  const bool live = 16 * wave < m;       // this wave has columns of X
 
-  // X(gi, 16 wave + lr') = sum_k Gi(gi, P_k) W(k, 16 wave + lr'): A operand lane = row + 16 k,
-  // B operand lane = column + 16 k, 8 k-steps of 4
-  cplx xa[FL_K / 4], xb[FL_K / 4];
+  // X(gi, 16 wave + lr') = sum_k Gi(gi, P_k) W(k, 16 wave + lr')
+  cplx xa[RF_K / 4], xb[RF_K / 4];
 #pragma unroll
-  for (int u = 0; u < FL_K / 4; ++u) {
+  for (int u = 0; u < RF_K / 4; ++u) {
     const int k = 4 * u + lk;
-    const int P = pa[u];
-    xa[u] = (k < m && row_ok) ? Gi[gi + (long long)P * n] : make_double2(0.0, 0.0);
-    xb[u] = k < m ? W[k + (long long)(16 * wave + lr) * FL_K] : make_double2(0.0, 0.0);
+    xa[u] = (live && k < m && row_ok) ? Gi[gi + (long long)pa[u] * n] : make_double2(0.0, 0.0);
+    xb[u] = (live && k < m) ? W[k + (long long)(16 * wave + lr) * CHAIN_W_LD] : make_double2(0.0, 0.0);
   }
-  // this wave's half of the rank-m product: Yhat(gj, k) for k in [16 wave, 16 wave + 16)
+  // Yhat(gj, k) for k in [16 wave, 16 wave + 16)
   cplx yb[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int k = 16 * wave + 4 * u + lk;
     yb[u] = make_double2(0.0, 0.0);
     if (k < m && col_ok) {
-      const int P = py[u];
-      const cplx v = Gi[P + (long long)gj * n];
-      yb[u] = make_double2((gj == P ? 1.0 : 0.0) - v.x, -v.y);
+      const cplx v = Gi[py[u] + (long long)gj * n];
+      yb[u] = make_double2((gj == py[u] ? 1.0 : 0.0) - v.x, -v.y);
     }
   }
-  // the tile of Gi in the MFMA result layout (wave 0 adds it)
+  // the tile of Gi in the layout of the product (wave 0 adds it)
   cplx gt[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1004,56 +999,63 @@ __global__ __launch_bounds__(128, 2) void round_flush_kernel(const cplx* __restr
     gt[r] = (wave == 0 && ri < n && col_ok) ? Gi[ri + (long long)gj * n] : make_double2(0.0, 0.0);
   }
 
-  v4d xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0};
+  if (live) {
+    v4d xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0}, xt = {0, 0, 0, 0};
 #pragma unroll
-  for (int u = 0; u < FL_K / 4; ++u) {
-    xr = M::mac(xa[u].x, xb[u].x, xr);
-    xi = M::mac(xa[u].x, xb[u].y, xi);
-    xr = M::mac(-xa[u].y, xb[u].y, xr);
-    xi = M::mac(xa[u].y, xb[u].x, xi);
-  }
+    for (int u = 0; u < RF_K / 4; ++u) {
+      if (16 * (u >> 2) < m) {
+        xr = M::mac(xa[u].x, xb[u].x, xr);
+        xt = M::mac(xa[u].y, xb[u].y, xt);
+        xi = M::mac(xa[u].x + xa[u].y, xb[u].x + xb[u].y, xi);
+      }
+    }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) Xs[M::row(r, lk)][16 * wave + lr] = make_double2(xr[r], xi[r]);
-  __syncthreads();
-
-  v4d gr = {0, 0, 0, 0}, gim = {0, 0, 0, 0};
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const cplx a = Xs[lr][16 * wave + 4 * u + lk];
-    gr = M::mac(a.x, yb[u].x, gr);
-    gim = M::mac(a.x, yb[u].y, gim);
-    gr = M::mac(-a.y, yb[u].y, gr);
-    gim = M::mac(a.y, yb[u].x, gim);
-  }
-  if (wave == 1) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[M::row(r, lk) + RF_T * lr] = make_double2(gr[r], gim[r]);
+    for (int r = 0; r < 4; ++r) Xs[M::row(r, lk)][16 * wave + lr] = make_double2(xr[r] - xt[r], xi[r] - xr[r] - xt[r]);
   }
   __syncthreads();
-  if (wave == 1 || !col_ok) return;
+  v4d gr = {0, 0, 0, 0}, gim = {0, 0, 0, 0}, gt2 = {0, 0, 0, 0};
+  if (live) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const cplx a = Xs[lr][16 * wave + 4 * u + lk];
+      gr = M::mac(a.x, yb[u].x, gr);
+      gt2 = M::mac(a.y, yb[u].y, gt2);
+      gim = M::mac(a.x + a.y, yb[u].x + yb[u].y, gim);
+    }
+    if (wave > 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave - 1][M::row(r, lk) + RF_T * lr] = make_double2(gr[r] - gt2[r], gim[r] - gr[r] - gt2[r]);
+    }
+  }
+  __syncthreads();
+  if (wave > 0 || !col_ok) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int ri = i0 + M::row(r, lk);
     if (ri >= n) continue;
-    const cplx h = red[M::row(r, lk) + RF_T * lr];
-    Go[ri + (long long)gj * n] = make_double2(gt[r].x + (gr[r] + h.x), gt[r].y + (gim[r] + h.y));
+    cplx v = make_double2(gr[r] - gt2[r], gim[r] - gr[r] - gt2[r]);
+#pragma unroll
+    for (int w = 1; w < RF_W; ++w)
+      if (16 * w < m) v = cadd(v, red[w - 1][M::row(r, lk) + RF_T * lr]);
+    Go[ri + (long long)gj * n] = cadd(gt[r], v);
   }
 }
 
 int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* W, const int* amap, const int* mdev, int n, int kmax,
                        int nchain, long long cs, hipStream_t s) {
-  if (kmax < 1 || kmax > FL_K) { alfq_set_error("round flush: rank outside [1, 32]"); return ST_GENERIC; }
+  if (kmax < 1 || kmax > CHAIN_BLOCK_KMAX) { alfq_set_error("round flush: rank outside the block kernel's depth"); return ST_GENERIC; }
   if (nchain < 1 || nchain > 65535 || n < 1) { alfq_set_error("round flush: bad batch"); return ST_GENERIC; }
   const unsigned t = (unsigned)cdivl(n, RF_T);
-  hipLaunchKernelGGL(round_flush_kernel, dim3(t, t, (unsigned)nchain), dim3(128), 0, s, Gi, Go, W, amap, mdev, n,
-                     kmax, cs);
+  hipLaunchKernelGGL(round_flush_kernel, dim3(t, t, (unsigned)nchain), dim3(64 * RF_W), 0, s, Gi, Go, W, amap, mdev,
+                     n, kmax, cs);
   HIP_OK(hipGetLastError());
   return ST_NONE;
 }
 
 int flush_launch(cplx* G, const cplx* X, const cplx* Y, const int* mdev, int n, int kmax, int nchain,
                  long long cs, hipStream_t s) {
-  if (kmax < 1 || kmax > FL_K) { alfq_set_error("flush: rank outside [1, 32]"); return ST_GENERIC; }
+  if (kmax < 1 || kmax > CHAIN_BLOCK_KMAX) { alfq_set_error("flush: rank outside the block kernel's depth"); return ST_GENERIC; }
   if (nchain < 1 || nchain > 65535) { alfq_set_error("flush: bad batch"); return ST_GENERIC; }
   const unsigned t = (unsigned)cdivl(n, FL_T);
   hipLaunchKernelGGL(flush_kernel, dim3(t, t, (unsigned)nchain), dim3(NT), 0, s, G, X, Y, mdev, n, kmax, cs);
