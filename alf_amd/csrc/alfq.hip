@@ -269,7 +269,7 @@ struct alfq_ctx {
   cplx* H = nullptr;
   cplx* X = nullptr;
   cplx* Y = nullptr;
-  cplx* Wk = nullptr;       // block kernel: W = C D^T of the last round (32 x 32)
+  cplx* CDk = nullptr;      // block kernel: C and D of the last round (32 x 32 each)
   int* amapk = nullptr;     // block kernel: sites of the last round's accepted flips
   ChainState* st = nullptr;
   DevScalars* sc = nullptr;
@@ -310,7 +310,7 @@ struct alfq_ctx {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   KTimer chain_timer;
   int rounds = 1 << 30;                  // chain rounds per slice (adapted per sweep)
-  bool round_fusion = true;              // one launch for a round's X product and flush (few chains)
+  bool round_fusion = true;              // one launch for a round's factors and flush (few chains)
   int* stat_dev = nullptr;               // 3 words per chain read after every sweep
   int* stat_host = nullptr;              // their pinned host copy
   bool visits_ready = false;             // the visits of the running pass are prepared
@@ -442,7 +442,7 @@ int metropolis_slice(alfq_ctx* c, int slice, int dir) {
   a.op_myexp = c->myexp; a.op_expalpha = c->expalpha; a.gama_ratio = c->gama_ratio;
   a.n_sun = c->n_sun;
   a.u = c->u; a.st = c->st;
-  a.W = c->Wk; a.amap = c->amapk;
+  a.CD = c->CDk; a.amap = c->amapk;
   a.cs = c->cs; a.nchain = c->B;
   a.lz = c->lz;
   a.uoff = dir > 0 ? c->uoff_up : c->uoff_dn;
@@ -459,34 +459,24 @@ int metropolis_slice(alfq_ctx* c, int slice, int dir) {
     hipLaunchKernelGGL(chain_reset_kernel, dim3(1, 1, c->B), dim3(1), 0, c->s, c->st, c->cs);
     HIP_OK(hipGetLastError());
   }
-  // X = G(:, A) W: the delayed-update columns of a round from its sites and W = C D^T.  When
-  // it runs on the direct-load kernel (few chains), that kernel also copies the rows A of G
-  // into Yhat, spread over its grid, in place of the block kernel's single workgroup.
-  GemmArgs gx = gemm_args(c->n, c->K, c->K, c->G, c->n, OP_N, true, c->Wk, CHAIN_W_LD, OP_N, true, c->X, c->n,
-                          ONE, ZERO);
-  gx.amap = c->amapk;
-  gx.kdev = &c->st->m;
-  gx.nchain = c->B;
-  gx.policy = c->gemm_policy;
-  a.yhat_external = reg_kernel && gemm_direct_path(gx) ? 1 : 0;
-  // few chains: X product and flush in one launch from G into the other G buffer (Gtmp is
+  // few chains: the whole flush of a round in one launch from G into the other G buffer (Gtmp is
   // free during the rounds), then the two swap.  Up to Ndim 256, where it was measured faster:
   // at Ndim 576 each 16 x 16 tile's gather of 32 rows of G costs more than the launch it saves
-  const bool fused = a.yhat_external && c->round_fusion && c->n <= 256;
-  if (a.yhat_external && !fused) gx.yhat = c->Y;
+  const bool fused = reg_kernel && c->round_fusion && c->n <= 256 && (long long)((c->n + 31) / 32) * c->B < 256;
   for (int r = 0; r < rounds; ++r) {
     a.first_round = (r == 0);
     a.final_round = (r == rounds - 1);
     a.G = c->G;
     if ((st = launch_chain(a, c->s, &c->chain_timer))) return st;
     if (fused) {
-      if ((st = round_flush_launch(c->G, c->Gtmp, c->Wk, c->amapk, &c->st->m, c->n, c->K, c->B, c->cs, c->s)))
+      if ((st = round_flush_launch(c->G, c->Gtmp, c->CDk, c->amapk, &c->st->m, c->n, c->K, c->B, c->cs, c->s)))
         return st;
       std::swap(c->G, c->Gtmp);
       continue;
     }
     if (reg_kernel) {
-      if ((st = gemm_c(c, gx))) return st;
+      if ((st = round_factors_launch(c->G, c->CDk, c->amapk, &c->st->m, c->X, c->Y, c->n, c->K, c->B, c->cs, c->s)))
+        return st;
     }
     // G += X Y^T with the rank read from the chain state
     const long long ftiles = (long long)((c->n + 63) / 64) * ((c->n + 63) / 64) * c->B;
@@ -1310,7 +1300,7 @@ void place_chain(alfq_ctx* c, ArenaLayout& ar, int nslot) {
   c->H = ar.take<cplx>(nn);
   c->X = ar.take<cplx>((size_t)n * CHAIN_KMAX);
   c->Y = ar.take<cplx>((size_t)n * CHAIN_KMAX);
-  c->Wk = ar.take<cplx>((size_t)CHAIN_KMAX * CHAIN_KMAX);
+  c->CDk = ar.take<cplx>((size_t)CHAIN_KMAX * CHAIN_KMAX);
   c->amapk = ar.take<int>(CHAIN_KMAX);
   c->st = ar.take<ChainState>(1);
   c->sc = ar.take<DevScalars>(1);

@@ -7,7 +7,7 @@
 
 #define CHAIN_KMAX 64   // largest delayed-update depth
 #define CHAIN_BLOCK_KMAX 32   // largest delayed-update depth of the block kernel
-#define CHAIN_W_LD 64   // leading dimension of the block kernel's W
+#define CHAIN_CD_LD 64   // leading dimension of the block kernel's C and D
 
 // Per-chain device state touched by the sequential Metropolis kernel.
 struct ChainState {
@@ -59,13 +59,11 @@ struct ChainArgs {
   int first_round;                // start of the slice: visit 0, rng base = current position
   int final_round;                // last scheduled round: flush in place instead of stopping at K
   ChainState* st;
-  // block kernel outputs for the flush G += (G(:, amap) W) Y^T: W (ld CHAIN_W_LD), site list
-  cplx* W; int* amap;
-  // nonzero: the round's X = G(:, amap) W product writes Yhat (GemmArgs::yhat), so the block
-  // kernel leaves Y alone except in its own in-place flush
-  int yhat_external;
+  // block kernel outputs for the flush G += (G(:, amap) C) (Yhat D)^T: C and, from column
+  // CHAIN_BLOCK_KMAX on, D (ld CHAIN_CD_LD), and the site list
+  cplx* CD; int* amap;
   // batches: byte stride between the chains' arenas; G, X, Y, f, the coupling tables
-  // (op_myexp, op_expalpha, gama_ratio), u, st, W and amap are per chain, op_site,
+  // (op_myexp, op_expalpha, gama_ratio), u, st, CD and amap are per chain, op_site,
   // op_type and uoff are shared
   long long cs;
   int nchain;

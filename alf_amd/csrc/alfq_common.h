@@ -164,10 +164,6 @@ struct GemmArgs {
   int slice;
   int hop_side;
   const void* ident;
-  // direct-load kernel only (gemm_direct_path): with amap set and a complex opA = A (OP_N),
-  // also write yhat(r, j) = delta(r, amap[j]) - A(amap[j], r) for r < M, j < K (ld M), the
-  // rows amap of A read before any later kernel changes A
-  cplx* yhat;
 };
 
 GemmArgs gemm_args(int M, int N, int K, const void* A, int lda, int opA, bool a_cplx,
@@ -178,14 +174,16 @@ int gemm_launch(const GemmArgs& g, hipStream_t s);
 // default, 1 the 64 x 64 kernel from one tile per CU, 2 never the 64 x 64 kernel, 3 the
 // direct-load kernel up to 512 tiles of 32 x 32.
 constexpr int GEMM_POLICIES = 4;
-// true when gemm_launch runs g on the direct-load kernel (the only one that honours yhat)
-bool gemm_direct_path(const GemmArgs& g);
 // G += X Y^T (all n x n / n x m, column-major, ld n) with the rank m read from *mdev and
 // clamped to kmax <= CHAIN_BLOCK_KMAX, for the nchain chains of a batch (pointers advance by cs bytes).
 int flush_launch(cplx* G, const cplx* X, const cplx* Y, const int* mdev, int n, int kmax, int nchain,
                  long long cs, hipStream_t s);
-// the round's X product and flush in one launch for a few chains: Go = Gi + (Gi(:, A) W) Yhat^T
-// with Yhat(c, j) = delta(c, amap[j]) - Gi(amap[j], c), rank m = *mdev <= kmax <= CHAIN_BLOCK_KMAX; W is
-// m x m with leading dimension CHAIN_W_LD; Gi and Go are different buffers.
-int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* W, const int* amap, const int* mdev, int n, int kmax,
+// The flush of a delayed-update round, Go = Gi + X Y^T with X = Gi(:, A) C and Y = Yhat D,
+// Yhat(c, j) = delta(c, amap[j]) - Gi(amap[j], c), rank m = *mdev <= kmax <= CHAIN_BLOCK_KMAX; CD holds
+// the m x m upper triangular C and, from column CHAIN_BLOCK_KMAX on, D, with leading dimension
+// CHAIN_CD_LD.  In one launch for a few chains (Gi and Go are different buffers), or X and Y (ld n)
+// alone, for a flush by flush_launch or gemm_launch.
+int round_factors_launch(const cplx* G, const cplx* CD, const int* amap, const int* mdev, cplx* X, cplx* Y, int n,
+                         int kmax, int nchain, long long cs, hipStream_t s);
+int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* CD, const int* amap, const int* mdev, int n, int kmax,
                        int nchain, long long cs, hipStream_t s);

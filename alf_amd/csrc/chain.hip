@@ -269,22 +269,26 @@ __global__ __launch_bounds__(256) void chain_kernel(ChainArgs a) {
 //
 // Full columns and rows of G are never formed here.  With A = (P_0, P_1, ...) the sites of
 // the round's accepted flips in order, G the Green's function at the start of the round and
-// Yhat(:, j) = e_{P_j} - G(P_j, :)^T, the current one is G_cur = G + G(:, A) W Yhat^T with
-// W m x m.  A block of flips extends W to W + Cn Dn^T, whose new columns are
-//   Cn(:, j) = -x_j (e_j + T2(:, p_j) + sum_{i<j} Cn(:, i) w_i(p_j)),   T2 = W Yhat[S]^T,
-//   Dn(:, j) =        e_j - T1(p_j, :)^T - sum_{i<j} Dn(:, i) u_i(p_j), T1 = G[S, A] W
-// (i, j over the block's flips), and the block starts from g = G[S, S] + T1 Yhat[S]^T.  T1, T2,
-// g and the update of W are on the matrix cores, and W is the only table that the round keeps.
-// W's tiles stay in the accumulators of the waves that own them; for T1 and T2 they are copied to
-// LDS, over the tables of the visits.  At the end the kernel leaves W and the site list A; the
-// flush is G += (G(:, A) W) Yhat^T over the device.
+// Yhat(:, j) = e_{P_j} - G(P_j, :)^T, the current one is G_cur = G + X Y^T with
+//   X = G(:, A) C,   Y = Yhat D,
+// C and D m x m and upper triangular, kept in LDS.  A block starts from g = G[S, S] + X[S] Y[S]^T,
+// X[S] = G[S, A] C, Y[S] = Yhat[S, A] D, and its flips add the columns
+//   C(:, m + j) = -x_j (e_j + T2(:, p_j) + sum_{i<j} C(:, m + i) w_i(p_j)),  T2 = C Y[S]^T,
+//   D(:, m + j) =        e_j - T1(p_j, :)^T - sum_{i<j} D(:, m + i) u_i(p_j), T1 = X[S] D^T
+// (i, j over the block's flips).  The four products are on the matrix cores.  At the end the
+// kernel leaves C, D and the site list A; the flush over the device is G += X Y^T.
+// One table W = C D^T (m x m) with G_cur = G + G(:, A) W Yhat^T, extended by each block to
+// W + Cn Dn^T, would save two of the block's products and one of the flush, but X and Y are of the
+// size of G's columns and rows, where W's entries are some 30 times as large and cancel in what is
+// formed from them: one slice's 32 flips left 7.8e-14 of G as error (C and D here and W in the
+// flush 3.7e-14, C and D throughout 2.1e-14), and G after ten slices was 3 to 6 times as far off.
 //
 // What bounds it: the chain of decisions, so the instructions and waits per accepted flip.  One
 // wave decides (no barrier inside a block), left-looking: lanes 0..31 hold column p of g, lanes
 // 32..63 row p, each formed from the block-start g and the block's earlier u_i, w_i in LDS, so a
 // flip costs one LDS round trip and a dot product over the block's flips instead of an update of
 // all of g by four waves between barriers; lane v keeps g(v, v) of its visit.  Two more waves
-// follow it flip by flip through flags in LDS and form the columns Cn and Dn (row l of W in
+// follow it flip by flip through flags in LDS and form the new columns of C and D (row l in
 // lane l), and a fourth fetches the next block's visit records, so that a block ends when its
 // last decision does.
 constexpr int SB_V = 32;    // visits per block: g is SB_V x SB_V
@@ -292,14 +296,12 @@ constexpr int SB_A = 16;    // accepted flips per block
 constexpr int SB_K = CHAIN_BLOCK_KMAX;   // accepted flips per round (delayed-update depth)
 constexpr int SB_T = 512;   // threads: 8 waves, two MFMA streams per SIMD
 constexpr int SB_W = SB_T / 64;
-constexpr int SB_M = (SB_K + 15) / 16;   // 16-wide tiles of W
+constexpr int SB_M = (SB_K + 15) / 16;   // 16-wide tiles of C and D
 constexpr int SB_PS = SB_V + 1;          // row pitch of the tables indexed by the block's sites
-constexpr int SB_PW = SB_K + 1;          // row pitch of W
-constexpr int SB_PL = SB_K + 1;          // row pitch of Cn, Dn (index l of W)
-constexpr int SB_TW = (SB_M * SB_M + SB_W - 1) / SB_W;   // tiles of W per wave
-static_assert((2 * SB_A - 1) * SB_PL + 16 * SB_M <= SB_K * SB_PS, "Cn and Dn lie over Yhat[S, A]");
-static_assert(SB_K <= CHAIN_W_LD, "W is stored with CHAIN_W_LD as leading dimension");
-static_assert(SB_K % 4 == 0 && 16 * SB_M <= 64, "row l of Cn and Dn is lane l of a wave");
+constexpr int SB_PL = SB_K + 1;          // row pitch of C and D
+static_assert(2 * SB_K <= CHAIN_CD_LD, "C beside D in a square of CHAIN_CD_LD");
+static_assert((SB_K & (SB_K - 1)) == 0, "indexes into C and D by masks");
+static_assert(SB_K == 16 * SB_M && SB_K <= 64, "whole tiles of C and D, row l in lane l of a wave");
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
@@ -329,24 +331,27 @@ __device__ __forceinline__ void both_halves(double v, double& low, double& high)
   high = __longlong_as_double(((long long)hi[1] << 32) | (long long)lo[1]);
 }
 
-// A 16 x 16 complex tile in three real accumulations: re = r - t, im = i - r - t
-struct Tile3 {
+// A 16 x 16 complex tile in four real products.  (Three, with im = (ar + ai)(br + bi) - re parts,
+// leave the imaginary parts the rounding of the real ones: the error of G over ten slices was
+// 1.15 times as large.)
+struct CTile {
   v4d r = {0, 0, 0, 0}, i = {0, 0, 0, 0}, t = {0, 0, 0, 0};
   __device__ __forceinline__ void mac(cplx a, cplx b) {
     r = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, r, 0, 0, 0);
+    i = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, i, 0, 0, 0);
     t = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, t, 0, 0, 0);
-    i = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x + a.y, b.x + b.y, i, 0, 0, 0);
+    i = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, i, 0, 0, 0);
   }
-  __device__ __forceinline__ cplx get(int q) const { return make_double2(r[q] - t[q], i[q] - r[q] - t[q]); }
+  __device__ __forceinline__ cplx get(int q) const { return make_double2(r[q] - t[q], i[q]); }
 };
-// tile += sum over k < kn (a multiple of 4) of fa(k + lk) fb(k + lk), lk = lane / 16: the next
+// tile += sum over k0 <= k < kn (multiples of 4) of fa(k + lk) fb(k + lk), lk = lane / 16: the next
 // step's operands are read while this step's products issue.  Register q of a lane holds the
 // entry of fa's index 4 q + lane / 16 and fb's index lane % 16.
 template <class FA, class FB>
-__device__ __forceinline__ void tile_mac(Tile3& c, int kn, int lk, FA fa, FB fb) {
-  if (kn <= 0) return;
-  cplx a = fa(lk), b = fb(lk);
-  for (int k = 4; k < kn; k += 4) {
+__device__ __forceinline__ void tile_mac(CTile& c, int k0, int kn, int lk, FA fa, FB fb) {
+  if (kn <= k0) return;
+  cplx a = fa(k0 + lk), b = fb(k0 + lk);
+  for (int k = k0 + 4; k < kn; k += 4) {
     const cplx an = fa(k + lk), bn = fb(k + lk);
     c.mac(a, b);
     a = an;
@@ -369,21 +374,20 @@ __device__ __forceinline__ void lds_order() { __asm__ volatile("" ::: "memory");
 // Bound by the serial chain of decisions: about 1240 clocks from one acceptance to the next (LDS
 // reads of the row and column, their dot product, the test, the ballot), 20 to 32 of them in a
 // launch.  Per launch for one chain of 16 x 16 22.8 us, where one rank-1 update of X, Y and g per
-// acceptance took 30.4 (its sweep 74.9 -> 65.0 ms); for 256 chains of 16 x 16 42.9 -> 38.7 us, of
-// 4 x 4 20.0 -> 14.3 us.  Rounds deeper than 32 lose in T1, T2 and W what they save in launches
-// (one chain's sweep at 40, 48 and 56: +2, +3 and +7 %).
+// acceptance took 30.4 (its sweep 74.9 -> 64.5 ms with the flush); for 256 chains of 4 x 4 20.0 ->
+// 14.3 us.  Rounds deeper than 32 lose in the products of a block what they save in launches (one
+// chain's sweep at 40, 48 and 56: +2, +3 and +7 %), and their error grows with the depth.
 // No array of this kernel may leave the registers: one that the compiler moves to LDS by thread
 // costs a read of the launch packet in host memory, 1.6 us and in a batch of 256 chains 8 us.
 __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
-  // W(l, j) at Wm[l][j] for T1 and T2; during the visits g(r, c) at gs[c][r] and u_i(s), w_i(s)
-  // at Tuw[i][s], Tuw[i][32 + s]
-  __shared__ cplx s_u[SB_K * SB_PW > SB_V * SB_PS + SB_A * 64 ? SB_K * SB_PW : SB_V * SB_PS + SB_A * 64];
-  cplx(*const Wm)[SB_PW] = (cplx(*)[SB_PW])s_u;
-  cplx(*const gs)[SB_PS] = (cplx(*)[SB_PS])s_u;
-  cplx(*const Tuw)[64] = (cplx(*)[64])(s_u + SB_V * SB_PS);
+  __shared__ cplx gs[SB_V][SB_PS];            // g(r, c) at [c][r]
+  __shared__ cplx Tuw[SB_A][64];              // u_i(s), w_i(s) at [i][s], [i][32 + s]
+  __shared__ cplx Cm[SB_K][SB_PL];            // C(l, j) at [j][l], l < SB_K, j < m
+  __shared__ cplx Dm[SB_K][SB_PL];            // D(l, j) at [j][l]
   __shared__ cplx Xa[SB_K][SB_PS];            // G(S_s, A_l) at [l][s], then T1(s, l)
-  __shared__ cplx Yh[SB_K][SB_PS];            // Yhat(S_s, l) at [l][s]; during the visits Cn, Dn
-  __shared__ cplx Wy[SB_K][SB_PS];            // T2(l, s) at [l][s]
+  __shared__ cplx Yh[SB_K][SB_PS];            // Yhat(S_s, l) at [l][s], then T2(l, s)
+  __shared__ cplx Xb[SB_K][SB_PS];            // X(S_s, j) at [j][s]
+  __shared__ cplx Yb[SB_K][SB_PS];            // Y(S_s, j) at [j][s]
   __shared__ BVisit vr[2][SB_V];
   __shared__ cplx s_x[SB_A];
   __shared__ int s_aP[SB_K];
@@ -391,8 +395,6 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
   // entry j: 1 + the index of flip j's site once flip j is in LDS, SB_FIN after the block's last
   __shared__ int s_pub[SB_A + 1];
   constexpr int SB_FIN = 0x100;
-  cplx* const Cn = &Yh[0][0];                 // Cn(l, j) at Cn[j * SB_PL + l], Dn alike
-  cplx* const Dn = Cn + SB_A * SB_PL;
 
   // (a wave's LDS operations complete in program order)
   auto publish = [&](int j, int what) {
@@ -409,7 +411,7 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
   a.f = chain_ptr(a.f, a.cs);
   a.rec = chain_ptr(a.rec, a.cs);
   a.st = chain_ptr(a.st, a.cs);
-  a.W = chain_ptr(a.W, a.cs);
+  a.CD = chain_ptr(a.CD, a.cs);
   a.amap = chain_ptr(a.amap, a.cs);
   ChainState* st = a.st;
   if (a.lz && a.slice >= a.lz[blockIdx.z]) {
@@ -487,40 +489,10 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
       }
     }
   };
-  // this wave's tiles of W, (tl, tj) = (t % SB_M, t / SB_M) for t = wave, wave + SB_W, ..: register
-  // q of a lane holds row 16 tl + 4 q + lane / 16 and column 16 tj + lane % 16; zero outside m x m
-  cplx wt[SB_TW][4];
-  auto zero_w = [&]() {
-#pragma unroll
-    for (int e = 0; e < SB_TW; ++e)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) wt[e][q] = make_double2(0.0, 0.0);
-  };
-  // f(e, row, column of register 0) for each of the wave's tiles that reaches into m x m
-  auto own_tiles = [&](auto&& f) {
-#pragma unroll
-    for (int e = 0; e < SB_TW; ++e) {
-      const int t = wave + SB_W * e, l0 = 16 * (t % SB_M), j0 = 16 * (t / SB_M);
-      if (l0 < m && j0 < m) f(e, l0, j0);
-    }
-  };
-  auto w_to_lds = [&]() {
-    const int ln = here(lane), lr = ln & 15, lk = ln >> 4;
-    own_tiles([&](int e, int l0, int j0) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int l = l0 + 4 * q + lk, j = j0 + lr;
-        if (l < SB_K && j < SB_K) Wm[l][j] = wt[e][q];
-      }
-    });
-  };
-
-  zero_w();
-  int cur = 1, mb = 0;
+  int cur = 1;
   bool cut = true;            // the records at vr[cur ^ 1] are not those of the visits from pos on
   while (true) {
-    // ---- the end of the block before and the start of the next: its sites' rows and columns of
-    // G are in flight while W += Cn Dn^T over the m x m corner goes into the tiles and to LDS ----
+    // ---- the next block: its sites' rows and columns of G are on their way ----
     const bool more = !stopped && pos < a.n_op && (m < kmax || a.final_round);
     cplx gss[4], gsa[NE], gas[NE];
     if (more) {
@@ -531,30 +503,20 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
       cur ^= 1;
       gather(vr[cur], a.n_op - pos < SB_V ? a.n_op - pos : SB_V, gss, gsa, gas);
     }
-    if (mb > 0) {
-      const int mb4 = (mb + 3) & ~3, ln = here(lane), lr = ln & 15, lk = ln >> 4;
-      own_tiles([&](int e, int l0, int j0) {
-        Tile3 c;
-        tile_mac(c, mb4, lk, [&](int i) { return Cn[i * SB_PL + l0 + lr]; },
-                 [&](int i) { return Dn[i * SB_PL + j0 + lr]; });
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (l0 + 4 * q + lk < m && j0 + lr < m) wt[e][q] = cadd(wt[e][q], c.get(q));
-      });
-    }
     if (!more) break;
-    w_to_lds();
-    __syncthreads();   // the block's tables are free and W is complete
     if (m >= kmax) {
-      // last round of the slice and the round is full: G += (G(:, A) W) Yhat^T in place
+      // last round of the slice and the round is full: G += X Y^T in place
       for (int r = tid; r < n; r += SB_T) {
         for (int j = 0; j < m; ++j) {
-          const int P = s_aP[j];
-          const cplx g = a.G[P + (long long)r * n];
-          a.Y[r + (long long)j * n] = make_double2((r == P ? 1.0 : 0.0) - g.x, -g.y);
-          cplx acc = make_double2(0.0, 0.0);
-          for (int l = 0; l < m; ++l) acc = cfma(a.G[r + (long long)s_aP[l] * n], Wm[l][j], acc);
-          a.X[r + (long long)j * n] = acc;
+          cplx x = make_double2(0.0, 0.0), y = make_double2(0.0, 0.0);
+          for (int l = 0; l <= j; ++l) {
+            const int P = s_aP[l];
+            const cplx g = a.G[P + (long long)r * n];
+            x = cfma(a.G[r + (long long)P * n], Cm[j][l], x);
+            y = cfma(make_double2((r == P ? 1.0 : 0.0) - g.x, -g.y), Dm[j][l], y);
+          }
+          a.X[r + (long long)j * n] = x;
+          a.Y[r + (long long)j * n] = y;
         }
       }
       __syncthreads();
@@ -566,13 +528,14 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
         }
       }
       m = 0;
-      zero_w();
       __syncthreads();
       gather(vr[cur], a.n_op - pos < SB_V ? a.n_op - pos : SB_V, gss, gsa, gas);
     }
     const int nb = a.n_op - pos < SB_V ? a.n_op - pos : SB_V;
     const int m4 = (m + 3) & ~3, mt = (m + 15) >> 4;
     const BVisit* const vc = vr[cur];
+    for (int e = here(tid); e < SB_A * 64; e += SB_T) (&Tuw[0][0])[e] = make_double2(0.0, 0.0);
+    if (tid <= SB_A) s_pub[tid] = 0;
     if (m > 0) {
       // ---- G[S, A] and Yhat[S, A] ----
       const int ln = here(lane), lr = ln & 15, lk = ln >> 4, td = here(tid);
@@ -589,59 +552,44 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
         }
       }
       __syncthreads();
-      // ---- T1 = G[S, A] W in place of G[S, A] (waves 0 .. 3), T2 = W Yhat[S, A]^T (4 .. 7):
-      //      tile t covers sites 16 (t % 2) and rows or columns 16 (t / 2) of W ----
-      constexpr int NT1 = (2 * SB_M + 3) / 4;
-      cplx t1[NT1][4];
+      // ---- X[S] = G[S, A] C (waves 0 .. 3) and Y[S] = Yhat[S, A] D (4 .. 7): tile t covers sites
+      //      16 (t % 2) and columns 16 (t / 2) of C or D, which are zero below the diagonal ----
+      for (int t = wave & 3; t < 2 * mt; t += 4) {
+        const int sc = 16 * (t & 1) + lr, j0 = 16 * (t >> 1), kn = m4 < j0 + 16 ? m4 : j0 + 16;
+        CTile c;
+        if (wave < 4)
+          tile_mac(c, 0, kn, lk, [&](int k) { return Cm[j0 + lr][k]; }, [&](int k) { return Xa[k][sc]; });
+        else
+          tile_mac(c, 0, kn, lk, [&](int k) { return Dm[j0 + lr][k]; }, [&](int k) { return Yh[k][sc]; });
+        cplx(*const out)[SB_PS] = wave < 4 ? Xb : Yb;
 #pragma unroll
-      for (int q = 0; q < NT1; ++q) {
-        const int t = (wave & 3) + 4 * q;
-        if (t < 2 * mt) {
-          const int sc = 16 * (t & 1) + lr, j = 16 * (t >> 1) + lr;
-          const int jc = j < SB_K ? j : SB_K - 1;
-          Tile3 c;
-          if (wave < 4) {
-            tile_mac(c, m4, lk, [&](int k) { return Wm[k][jc]; }, [&](int k) { return Xa[k][sc]; });
-#pragma unroll
-            for (int r = 0; r < 4; ++r) t1[q][r] = c.get(r);
-          } else {
-            tile_mac(c, m4, lk, [&](int k) { return Wm[jc][k]; }, [&](int k) { return Yh[k][sc]; });
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int l = 16 * (t >> 1) + 4 * r + lk;
-              if (l < SB_K) Wy[l][sc] = c.get(r);
-            }
-          }
-        }
-      }
-      __syncthreads();
-      if (wave < 4) {
-#pragma unroll
-        for (int q = 0; q < NT1; ++q) {
-          const int t = wave + 4 * q;
-          if (t < 2 * mt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int j = 16 * (t >> 1) + 4 * r + lk;
-              if (j < SB_K) Xa[j][16 * (t & 1) + lr] = t1[q][r];
-            }
-          }
-        }
+        for (int r = 0; r < 4; ++r) out[j0 + 4 * r + lk][sc] = c.get(r);
       }
       __syncthreads();
     }
-    // ---- g = G[S, S] + T1 Yhat[S, A]^T ----
+    // ---- g = G[S, S] + X[S] Y[S]^T (waves 0 .. 3); T1 = X[S] D^T and T2 = C Y[S]^T (4 .. 7) ----
     if (wave < 4) {
       const int ln = here(lane), lr = ln & 15, lk = ln >> 4;
       const int r = 16 * (wave & 1) + lr, c0 = 16 * (wave >> 1);
-      Tile3 c;
-      tile_mac(c, m4, lk, [&](int k) { return Yh[k][c0 + lr]; }, [&](int k) { return Xa[k][r]; });
+      CTile c;
+      tile_mac(c, 0, m4, lk, [&](int k) { return Yb[k][c0 + lr]; }, [&](int k) { return Xb[k][r]; });
 #pragma unroll
       for (int q = 0; q < 4; ++q) gs[c0 + 4 * q + lk][r] = cadd(gss[q], c.get(q));
     } else {
-      // (T1 and T2 have read W, which lies below)
-      for (int e = here(tid) - 256; e < SB_A * 64; e += SB_T - 256) (&Tuw[0][0])[e] = make_double2(0.0, 0.0);
-      if (tid - 256 <= SB_A) s_pub[tid - 256] = 0;
+      const int ln = here(lane), lr = ln & 15, lk = ln >> 4;
+      for (int t = wave & 3; t < 4 * mt; t += 4) {
+        // rows l0 .. l0 + 15 of C and D begin at column l0
+        const int sc = 16 * (t & 1) + lr, l0 = 16 * (t >> 2);
+        const bool t1 = (t & 2) == 0;
+        CTile c;
+        if (t1)
+          tile_mac(c, l0, m4, lk, [&](int k) { return Dm[k][l0 + lr]; }, [&](int k) { return Xb[k][sc]; });
+        else
+          tile_mac(c, l0, m4, lk, [&](int k) { return Cm[k][l0 + lr]; }, [&](int k) { return Yb[k][sc]; });
+        cplx(*const out)[SB_PS] = t1 ? Xa : Yh;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[l0 + 4 * r + lk][sc] = c.get(r);
+      }
     }
     __syncthreads();
 
@@ -768,12 +716,12 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
         publish(mb, SB_FIN);
       }
     } else if (wave <= 2) {
-      // ---- columns Cn (wave 1) and Dn (wave 2), row l of W in lane l ----
+      // ---- the new columns of C (wave 1) and D (wave 2), row l in lane l ----
       const bool isc = wave == 1;
       const int l = here(lane), lc = l < SB_K ? l : SB_K - 1;
-      const cplx* const T = isc ? &Wy[lc][0] : &Xa[lc][0];   // T2(l, :) / T1(:, l)
+      const cplx* const T = isc ? &Yh[lc][0] : &Xa[lc][0];   // T2(l, :) / T1(:, l)
       const cplx* const N = &Tuw[0][isc ? 32 : 0];           // w_i(p) / u_i(p)
-      cplx* const out = isc ? Cn : Dn;
+      cplx* const out = isc ? &Cm[m][0] : &Dm[m][0];
       int j = 0;
       while (true) {
         const int pub = __hip_atomic_load(&s_pub[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -807,15 +755,15 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
         if (l < SB_K) out[j * SB_PL + l] = r;
         ++j;
       }
-      // zero up to a whole k-step of the product below
-      for (; j & 3; ++j)
+      // zero up to a whole k-step of the products
+      for (; (m + j) & 3; ++j)
         if (l < SB_K) out[j * SB_PL + l] = make_double2(0.0, 0.0);
     } else if (wave == SB_W - 1) {
       // the records of the block after this one, if this one is not cut short
       records(pos + nb, cur ^ 1);
     }
     __syncthreads();
-    mb = s_mb;
+    const int mb = s_mb;
     const int k = s_k;
     stopped = s_stopped != 0;
     m += mb;
@@ -824,24 +772,11 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
     cut = k < nb;                            // the next block does not start where the records do
     pos += k;
   }
-  // ---- the round's flush operands: W (zero up to whole tiles of 16), the site list, Yhat ----
-  own_tiles([&](int e, int l0, int j0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a.W[l0 + 4 * q + lk + CHAIN_W_LD * (j0 + lr)] = wt[e][q];
-  });
-  if (!a.yhat_external) {
-    // Yhat(r, j) = delta(r, P_j) - G(P_j, r)
-    for (int r = tid; r < n; r += SB_T) {
-      for (int j0 = 0; j0 < m; j0 += 8) {
-        cplx gv[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) gv[t] = a.G[(j0 + t < m ? s_aP[j0 + t] : 0) + (long long)r * n];
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-          if (j0 + t < m)
-            a.Y[r + (long long)(j0 + t) * n] = make_double2((r == s_aP[j0 + t] ? 1.0 : 0.0) - gv[t].x, -gv[t].y);
-      }
-    }
+  // ---- the round's flush operands: C, D and the site list ----
+  for (int e = tid; e < SB_K * m; e += SB_T) {
+    const int l = e & (SB_K - 1), j = e / SB_K;
+    a.CD[l + CHAIN_CD_LD * j] = Cm[j][l];
+    a.CD[l + CHAIN_CD_LD * (CHAIN_BLOCK_KMAX + j)] = Dm[j][l];
   }
   if (tid < CHAIN_KMAX) a.amap[tid] = tid < m ? s_aP[tid] : 0;
   if (tid == 0) {

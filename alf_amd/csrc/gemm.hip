@@ -63,13 +63,12 @@ __device__ __forceinline__ bool chain_operands(GemmArgs& g, int bz) {
   g.A = mv(g.A); g.B = mv(g.B); g.C = (void*)mv((const char*)g.C);
   g.rs = mv(g.rs); g.cs = mv(g.cs); g.bs = mv(g.bs); g.rs_real = mv(g.rs_real);
   g.amap = mv(g.amap); g.bmap = mv(g.bmap); g.kdev = mv(g.kdev);
-  g.yhat = mv(g.yhat);
   if (g.lz && g.slice >= g.lz[bz / (g.batch > 1 ? g.batch : 1)]) {
     if (g.hop_side == 1) g.A = g.ident;
     else if (g.hop_side == 2) g.B = g.ident;
     // the identity is K x K: M = K when it is opA, N = K when it is opB
     return ((g.hop_side == 1 && g.M == g.K) || (g.hop_side == 2 && g.N == g.K)) && g.batch <= 1 && !g.amap &&
-           !g.bmap && !g.kdev && !g.yhat;
+           !g.bmap && !g.kdev;
   }
   return false;
 }
@@ -769,19 +768,6 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_direct_kernel(GemmArgs g) {
     const int kd = *g.kdev;
     K = kd < K ? kd : K;
   }
-  if (A_CPLX && g.yhat && g.amap) {
-    // the side copy of rows amap of A, spread over every thread of the grid
-    const int nwg = gridDim.x * gridDim.y;
-    const long long total = (long long)g.M * (K > 0 ? K : 0);
-    const cplx* Ag = (const cplx*)g.A;
-    for (long long e = (long long)(blockIdx.x + gridDim.x * blockIdx.y) * blockDim.x + tid; e < total;
-         e += (long long)nwg * blockDim.x) {
-      const int r = (int)(e % g.M), j = (int)(e / g.M);
-      const int P = g.amap[j];
-      const cplx v = Ag[P + (long long)r * g.lda];
-      g.yhat[e] = make_double2((r == P ? 1.0 : 0.0) - v.x, -v.y);
-    }
-  }
   if (K <= 0 && g.beta.x == 1.0 && g.beta.y == 0.0) return;  // nothing to add
   const double* Ar = (const double*)g.A;
   const cplx* Ac = (const cplx*)g.A;
@@ -933,121 +919,177 @@ void launch_direct(const GemmArgs& g, hipStream_t s) {
 }
 }  // namespace
 
-// The end of a delayed-update round for a few chains, in one launch:
-//   Go = Gi + (Gi(:, A) W) Yhat^T,   Yhat(c, j) = delta(c, P_j) - Gi(P_j, c),
-// A = (P_0 .. P_{m-1}) the round's accepted sites, W m x m with leading dimension CHAIN_W_LD,
-// m = *mdev <= CHAIN_BLOCK_KMAX.  Gi is only read and Go only written (two buffers), so a
-// workgroup can gather the columns A and rows A of Gi that it needs while others write their
-// tiles.  A workgroup of RF_W waves owns a 16 x 16 tile: wave w forms columns 16 w .. 16 w + 15 of
-// its rows of X = Gi(:, A) W, then takes the same 16 of the rank-m product, and the parts are
-// added through LDS.  Latency-bound: every global load of the tile is issued before the first MFMA,
-// and the sites are read beside m so that the gathers wait for one load.
+// ---- the flush of a delayed-update round -------------------------------------------------------
+//   Go = Gi + X Y^T,   X = Gi(:, A) C,   Y = Yhat D,   Yhat(c, j) = delta(c, P_j) - Gi(P_j, c),
+// A = (P_0 .. P_{m-1}) the round's accepted sites, CD the m x m upper triangular C and, from column
+// CHAIN_BLOCK_KMAX on, D, with leading dimension CHAIN_CD_LD, m = *mdev <= CHAIN_BLOCK_KMAX.
+// All products are four real ones: with three, the imaginary parts get the rounding of the real ones.
 constexpr int RF_T = 16, RF_W = (CHAIN_BLOCK_KMAX + 15) / 16, RF_K = 16 * RF_W;
-__global__ __launch_bounds__(64 * RF_W, 2) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
-                                                                  const cplx* __restrict__ W,
-                                                                  const int* __restrict__ amap, const int* mdev,
-                                                                  int n, int kmax, long long cs) {
+
+// One wave's 16 rows r0 .. and columns 16 w .. 16 w + 15 of X or (isy) Y: register q of a lane holds
+// column 16 w + 4 q + lane / 16 of row r0 + lane % 16, which is gr; live: the wave has columns
+// below m.  Every global load is issued before the first MFMA, and the sites are read beside m so
+// that the gathers wait for one load.  C and D are zero below row 16 w + 15.
+struct RoundFactor {
+  cplx ga[RF_K / 4], cd[RF_K / 4];
+  v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0}, t = {0, 0, 0, 0};
+  // (the sites' buffer holds CHAIN_KMAX >= RF_K entries)
+  __device__ __forceinline__ void load(const cplx* __restrict__ G, const cplx* __restrict__ CD, const int (&pa)[RF_K / 4],
+                                       int m, int n, int gr, int w, bool isy) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int u = 0; u < RF_K / 4; ++u) {
+      const int k = 4 * u + lk;
+      const bool in = 16 * w < m && k < m && u < 4 * (w + 1);
+      ga[u] = (in && gr < n) ? G[isy ? pa[u] + (long long)gr * n : gr + (long long)pa[u] * n] : make_double2(0.0, 0.0);
+      cd[u] = (in && 16 * w + lr < m) ? CD[k + (long long)((isy ? CHAIN_BLOCK_KMAX : 0) + 16 * w + lr) * CHAIN_CD_LD]
+                                      : make_double2(0.0, 0.0);
+      if (isy && in && gr < n) ga[u] = make_double2((gr == pa[u] ? 1.0 : 0.0) - ga[u].x, -ga[u].y);
+    }
+  }
+  __device__ __forceinline__ void mul(int w) {
+    typedef Mma<false> M;
+#pragma unroll
+    for (int u = 0; u < RF_K / 4; ++u) {
+      if (u < 4 * (w + 1)) {
+        re = M::mac(cd[u].x, ga[u].x, re);
+        im = M::mac(cd[u].x, ga[u].y, im);
+        t = M::mac(cd[u].y, ga[u].y, t);
+        im = M::mac(cd[u].y, ga[u].x, im);
+      }
+    }
+  }
+  __device__ __forceinline__ cplx get(int q) const { return make_double2(re[q] - t[q], im[q]); }
+};
+
+// X and Y alone, for batches and for matrices whose tiles are too many for the kernel below: 16
+// rows to a workgroup, its waves as below.  The rows A of G are gathered here, over the device, and
+// not by the block kernel's one workgroup a chain.
+__global__ __launch_bounds__(128 * RF_W, 2) void round_factors_kernel(const cplx* __restrict__ G,
+                                                                     const cplx* __restrict__ CD,
+                                                                     const int* __restrict__ amap, const int* mdev,
+                                                                     cplx* __restrict__ X, cplx* __restrict__ Y,
+                                                                     int n, int kmax, long long cs) {
+  const int z = blockIdx.z;
+  G = chain_ptr_at(G, cs, z);
+  CD = chain_ptr_at(CD, cs, z);
+  amap = chain_ptr_at(amap, cs, z);
+  mdev = chain_ptr_at(mdev, cs, z);
+  X = chain_ptr_at(X, cs, z);
+  Y = chain_ptr_at(Y, cs, z);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lr = lane & 15, lk = lane >> 4;
+  const bool isy = wave >= RF_W;
+  const int w = isy ? wave - RF_W : wave;
+  const int gr = blockIdx.x * RF_T + lr;
+  int pa[RF_K / 4];
+#pragma unroll
+  for (int u = 0; u < RF_K / 4; ++u) pa[u] = amap[4 * u + lk];
+  int m = *mdev;
+  m = m < kmax ? m : kmax;
+  RoundFactor f;
+  f.load(G, CD, pa, m, n, gr, w, isy);
+  if (16 * w >= m) return;
+  f.mul(w);
+  cplx* const out = isy ? Y : X;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int j = 16 * w + 4 * q + lk;
+    if (j < m && gr < n) out[gr + (long long)j * n] = f.get(q);
+  }
+}
+
+// The whole flush for a few chains, in one launch.  Gi is only read and Go only written (two
+// buffers), so a workgroup can gather the columns A and rows A of Gi that it needs while others
+// write their tiles.  A workgroup owns a 16 x 16 tile: of its 2 RF_W waves the first half forms its
+// rows of X, the second its rows of Y, 16 columns each; then RF_W waves take 16 columns of the
+// rank-m product each, and the parts are added through LDS.  Latency-bound.
+__global__ __launch_bounds__(128 * RF_W, 2) void round_flush_kernel(const cplx* __restrict__ Gi, cplx* __restrict__ Go,
+                                                                   const cplx* __restrict__ CD,
+                                                                   const int* __restrict__ amap, const int* mdev,
+                                                                   int n, int kmax, long long cs) {
   typedef Mma<false> M;
-  __shared__ cplx Xs[RF_T][RF_K + 1];
+  __shared__ cplx XY[2][RF_K][RF_T + 1];   // X(i0 + r, j), Y(j0 + r, j) at [j][r]
   __shared__ cplx red[RF_W - 1][RF_T * RF_T];
   const int z = blockIdx.z;
   Gi = chain_ptr_at(Gi, cs, z);
   Go = chain_ptr_at(Go, cs, z);
-  W = chain_ptr_at(W, cs, z);
+  CD = chain_ptr_at(CD, cs, z);
   amap = chain_ptr_at(amap, cs, z);
   mdev = chain_ptr_at(mdev, cs, z);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
+  const bool isy = wave >= RF_W;
+  const int w = isy ? wave - RF_W : wave;
   const int i0 = blockIdx.x * RF_T, j0 = blockIdx.y * RF_T;
-  const int gi = i0 + lr, gj = j0 + lr;
-  const bool row_ok = gi < n, col_ok = gj < n;
-  // (the sites' buffer holds CHAIN_KMAX >= RF_K entries)
-  int pa[RF_K / 4], py[4];
+  const int gj = j0 + lr;
+  int pa[RF_K / 4];
 #pragma unroll
   for (int u = 0; u < RF_K / 4; ++u) pa[u] = amap[4 * u + lk];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) py[u] = amap[16 * wave + 4 * u + lk];
   int m = *mdev;
   m = m < kmax ? m : kmax;
   m = m > 0 ? m : 0;
-  const bool live = 16 * wave < m;       // this wave has columns of X
-
-  // X(gi, 16 wave + lr') = sum_k Gi(gi, P_k) W(k, 16 wave + lr')
-  cplx xa[RF_K / 4], xb[RF_K / 4];
-#pragma unroll
-  for (int u = 0; u < RF_K / 4; ++u) {
-    const int k = 4 * u + lk;
-    xa[u] = (live && k < m && row_ok) ? Gi[gi + (long long)pa[u] * n] : make_double2(0.0, 0.0);
-    xb[u] = (live && k < m) ? W[k + (long long)(16 * wave + lr) * CHAIN_W_LD] : make_double2(0.0, 0.0);
-  }
-  // Yhat(gj, k) for k in [16 wave, 16 wave + 16)
-  cplx yb[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int k = 16 * wave + 4 * u + lk;
-    yb[u] = make_double2(0.0, 0.0);
-    if (k < m && col_ok) {
-      const cplx v = Gi[py[u] + (long long)gj * n];
-      yb[u] = make_double2((gj == py[u] ? 1.0 : 0.0) - v.x, -v.y);
-    }
-  }
+  const bool live = 16 * w < m;
+  RoundFactor f;
+  f.load(Gi, CD, pa, m, n, isy ? gj : i0 + lr, w, isy);
   // the tile of Gi in the layout of the product (wave 0 adds it)
   cplx gt[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int ri = i0 + M::row(r, lk);
-    gt[r] = (wave == 0 && ri < n && col_ok) ? Gi[ri + (long long)gj * n] : make_double2(0.0, 0.0);
+    gt[r] = (wave == 0 && ri < n && gj < n) ? Gi[ri + (long long)gj * n] : make_double2(0.0, 0.0);
   }
-
   if (live) {
-    v4d xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0}, xt = {0, 0, 0, 0};
+    f.mul(w);
 #pragma unroll
-    for (int u = 0; u < RF_K / 4; ++u) {
-      if (16 * (u >> 2) < m) {
-        xr = M::mac(xa[u].x, xb[u].x, xr);
-        xt = M::mac(xa[u].y, xb[u].y, xt);
-        xi = M::mac(xa[u].x + xa[u].y, xb[u].x + xb[u].y, xi);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) Xs[M::row(r, lk)][16 * wave + lr] = make_double2(xr[r] - xt[r], xi[r] - xr[r] - xt[r]);
+    for (int q = 0; q < 4; ++q) XY[isy][16 * w + 4 * q + lk][lr] = f.get(q);
   }
   __syncthreads();
-  v4d gr = {0, 0, 0, 0}, gim = {0, 0, 0, 0}, gt2 = {0, 0, 0, 0};
-  if (live) {
+  v4d gre = {0, 0, 0, 0}, gim = {0, 0, 0, 0}, gt2 = {0, 0, 0, 0};
+  if (live && !isy) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const cplx a = Xs[lr][16 * wave + 4 * u + lk];
-      gr = M::mac(a.x, yb[u].x, gr);
-      gt2 = M::mac(a.y, yb[u].y, gt2);
-      gim = M::mac(a.x + a.y, yb[u].x + yb[u].y, gim);
+      const cplx a = XY[0][16 * w + 4 * u + lk][lr], b = XY[1][16 * w + 4 * u + lk][lr];
+      gre = M::mac(a.x, b.x, gre);
+      gim = M::mac(a.x, b.y, gim);
+      gt2 = M::mac(a.y, b.y, gt2);
+      gim = M::mac(a.y, b.x, gim);
     }
-    if (wave > 0) {
+    if (w > 0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[wave - 1][M::row(r, lk) + RF_T * lr] = make_double2(gr[r] - gt2[r], gim[r] - gr[r] - gt2[r]);
+      for (int r = 0; r < 4; ++r) red[w - 1][M::row(r, lk) + RF_T * lr] = make_double2(gre[r] - gt2[r], gim[r]);
     }
   }
   __syncthreads();
-  if (wave > 0 || !col_ok) return;
+  if (wave > 0 || gj >= n) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int ri = i0 + M::row(r, lk);
     if (ri >= n) continue;
-    cplx v = make_double2(gr[r] - gt2[r], gim[r] - gr[r] - gt2[r]);
+    cplx v = make_double2(gre[r] - gt2[r], gim[r]);
 #pragma unroll
-    for (int w = 1; w < RF_W; ++w)
-      if (16 * w < m) v = cadd(v, red[w - 1][M::row(r, lk) + RF_T * lr]);
+    for (int q = 1; q < RF_W; ++q)
+      if (16 * q < m) v = cadd(v, red[q - 1][M::row(r, lk) + RF_T * lr]);
     Go[ri + (long long)gj * n] = cadd(gt[r], v);
   }
 }
 
-int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* W, const int* amap, const int* mdev, int n, int kmax,
+int round_factors_launch(const cplx* G, const cplx* CD, const int* amap, const int* mdev, cplx* X, cplx* Y, int n,
+                         int kmax, int nchain, long long cs, hipStream_t s) {
+  if (kmax < 1 || kmax > CHAIN_BLOCK_KMAX) { alfq_set_error("round factors: rank outside the block kernel's depth"); return ST_GENERIC; }
+  if (nchain < 1 || nchain > 65535 || n < 1) { alfq_set_error("round factors: bad batch"); return ST_GENERIC; }
+  hipLaunchKernelGGL(round_factors_kernel, dim3((unsigned)cdivl(n, RF_T), 1, (unsigned)nchain), dim3(128 * RF_W), 0, s,
+                     G, CD, amap, mdev, X, Y, n, kmax, cs);
+  HIP_OK(hipGetLastError());
+  return ST_NONE;
+}
+
+int round_flush_launch(const cplx* Gi, cplx* Go, const cplx* CD, const int* amap, const int* mdev, int n, int kmax,
                        int nchain, long long cs, hipStream_t s) {
   if (kmax < 1 || kmax > CHAIN_BLOCK_KMAX) { alfq_set_error("round flush: rank outside the block kernel's depth"); return ST_GENERIC; }
   if (nchain < 1 || nchain > 65535 || n < 1) { alfq_set_error("round flush: bad batch"); return ST_GENERIC; }
   const unsigned t = (unsigned)cdivl(n, RF_T);
-  hipLaunchKernelGGL(round_flush_kernel, dim3(t, t, (unsigned)nchain), dim3(64 * RF_W), 0, s, Gi, Go, W, amap, mdev,
+  hipLaunchKernelGGL(round_flush_kernel, dim3(t, t, (unsigned)nchain), dim3(128 * RF_W), 0, s, Gi, Go, CD, amap, mdev,
                      n, kmax, cs);
   HIP_OK(hipGetLastError());
   return ST_NONE;
@@ -1110,17 +1152,13 @@ static const TilePolicy& tile_policy(const GemmArgs& g) {
   return kTilePolicy[(g.policy >= 0 && g.policy < GEMM_POLICIES) ? g.policy : 0];
 }
 
-bool gemm_direct_path(const GemmArgs& g) {
+static bool gemm_direct_path(const GemmArgs& g) {
   return g.M > 0 && g.N > 0 && cdivl(g.M, 32) * cdivl(g.N, 32) * (long long)gemm_zdim(g) < tile_policy(g).direct_below;
 }
 
 int gemm_launch(const GemmArgs& g, hipStream_t s) {
   if (g.M <= 0 || g.N <= 0) return ST_NONE;
   if (gemm_zdim(g) > 65535) { alfq_set_error("gemm_launch: batch too large"); return ST_GENERIC; }
-  if (g.yhat && !(gemm_direct_path(g) && g.amap && g.a_cplx && g.opA == OP_N && g.batch <= 1)) {
-    alfq_set_error("gemm_launch: the row copy yhat needs the direct kernel, a complex opA = A and amap");
-    return ST_GENERIC;
-  }
   const long long b = gemm_zdim(g);
   if (gemm_direct_path(g)) {
     // too few 32 x 32 tiles to fill the device: 16 x 16 tiles, K split over up to 8 waves

@@ -68,3 +68,26 @@ def test_rounds_follow_sequential_visits(rt, delay, n_sun, ops):
     assert c["NC_up"] == s.ctrl.NC_up and c["ACC_up"] == s.ctrl.ACC_up
     assert c["ACC_up"] > 0.2 * c["NC_up"]
     e.close()
+
+
+@pytest.mark.parametrize("L1,L2,delay", [(5, 4, 1), (5, 4, 15), (3, 11, 16), (7, 5, 17), (4, 12, 32)])
+def test_flush_of_a_round_in_one_launch_and_in_two(rt, L1, L2, delay):
+    """G after the slices of one interval with the factors X and Y of each round formed inside the
+    flush and by a kernel of their own: the same sums in another order, so 1e-12 of G.  (Depths
+    below, at and above 16 columns, Ndim with and without a remainder of 16.)"""
+    ham = hubbard(L1=L1, L2=L2, beta=0.6, nwrap=3, U=2.0)
+    f = fields_for(ham, 3)
+    got = []
+    for on in (1, 0):
+        e = rt.Engine(ham, delay=delay)
+        e.round_fusion(bool(on))
+        e.set_fields(f)
+        e.set_philox(11, 0)
+        e.init()
+        for nt in range(3):
+            e.wrapgrup(nt, e.get_phase())
+        got.append((e.get_green(), e.get_fields(), e.rng_position()))
+        e.close()
+    assert np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+    assert not np.array_equal(got[0][1], f)
+    assert rel(got[1][0], got[0][0]) < 1e-12
