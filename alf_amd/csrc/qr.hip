@@ -537,21 +537,62 @@ __global__ __launch_bounds__(PLT) void panel_lds_kernel(cplx* __restrict__ A, in
   }
 }
 
+// The reflector of a column: beta, tau and the scale of v for its leading element alpha and the
+// squared norm xs of the rest (zlarfg without the rescaling loop).  In the range where no square
+// under- or overflows, beta and 1 / beta come from one reciprocal square root and 1 / (alpha -
+// beta) from one reciprocal, both with Newton steps to full precision, instead of a square root
+// and three divisions one after another: the column's owner is the panel's critical path.
+__device__ __forceinline__ void reflector(cplx alpha, double xs, double& beta, cplx& tau, cplx& sc) {
+  tau = make_double2(0.0, 0.0);
+  sc = make_double2(1.0, 0.0);
+  beta = alpha.x;
+  if (xs == 0.0 && alpha.y == 0.0) return;
+  const double s = alpha.x * alpha.x + alpha.y * alpha.y + xs;
+  if (s > 1e-280 && s < 1e280) {
+    double r = __builtin_amdgcn_rsq(s);
+    r = fma(0.5 * r, fma(-s * r, r, 1.0), r);
+    r = fma(0.5 * r, fma(-s * r, r, 1.0), r);
+    double nrm = s * r;
+    nrm = fma(fma(-nrm, nrm, s), 0.5 * r, nrm);
+    beta = -copysign(nrm, alpha.x);
+    const double rb = -copysign(r, alpha.x), zx = alpha.x - beta, q = fma(zx, zx, alpha.y * alpha.y);
+    double iq = __builtin_amdgcn_rcp(q);
+    iq = fma(fma(-q, iq, 1.0), iq, iq);
+    iq = fma(fma(-q, iq, 1.0), iq, iq);
+    tau = make_double2(-zx * rb, -alpha.y * rb);
+    sc = make_double2(zx * iq, -alpha.y * iq);
+    return;
+  }
+  beta = -copysign(sqrt(s), alpha.x);
+  const double rb = 1.0 / beta;
+  tau = make_double2((beta - alpha.x) * rb, -alpha.y * rb);
+  // 1 / (alpha - beta) by Smith's scaling with one reciprocal
+  const double zx = alpha.x - beta, zy = alpha.y;
+  if (fabs(zx) >= fabs(zy)) {
+    const double r = zy / zx, id = 1.0 / (zx + r * zy);
+    sc = make_double2(id, -r * id);
+  } else {
+    const double r = zx / zy, id = 1.0 / (zy + r * zx);
+    sc = make_double2(r * id, -id);
+  }
+}
+
 // ---- panel factorisation with the panel resident in registers (rows <= 256) -----
 // Same contract as panel_kernel except that Y2 = V T is not formed here (qr_form_q
 // forms it with the GEMM).  1024 threads: the 32 lanes of half-wave c hold column c,
-// rows l, l + 32, ..., l + 224 (l = lane in the half-wave).  Column j's reflector is
+// rows l, l + 32, ... (l = lane in the half-wave), RPL of them: the launcher takes the least of 1, 2,
+// 4 and 8 that holds the rows, for a step costs the same for rows that are zero.  Column j's reflector is
 // formed by its own half-wave and handed to the others through a double-buffered LDS
 // vector, one barrier per column; columns right of j apply H^H in registers, columns
 // left of j (already final) use the step to accumulate the Gram entry v_c^H v_j.
 // T follows from T^-1 = striu(V^H V) + diag(1/tau) (the columnwise zlarft recurrence
 // T(0:j, j) = -tau_j T(0:j, 0:j) V^H v_j, inverted), by a fan-in solve per column,
 // and Y1 = V T^H is an MFMA product out of LDS.
-constexpr int RPL = 8;          // rows per lane: 256 rows
-constexpr int RP = 32 * RPL;
+constexpr int RP_MAX = 256;     // rows: up to 8 per lane
 
 __device__ __forceinline__ double hsum32(double v) { return half_sum(v); }
 
+template <int RPL>
 __global__ __launch_bounds__(1024) void panel_reg_kernel(cplx* __restrict__ A, int n, int k, int nb,
                                                          cplx* __restrict__ tau, cplx* __restrict__ Vw,
                                                          cplx* __restrict__ Y1w, cplx* __restrict__ Tw,
@@ -562,6 +603,7 @@ __global__ __launch_bounds__(1024) void panel_reg_kernel(cplx* __restrict__ A, i
   Y1w = chain_ptr(Y1w, cs);
   Tw = chain_ptr(Tw, cs);
   pdet = chain_ptr(pdet, cs);
+  constexpr int RP = 32 * RPL;
   extern __shared__ cplx smem[];      // loop: vbuf[2][RP]; afterwards: V[RP x 32], column-major
   __shared__ cplx s_S[32 * 32];       // Gram above the diagonal, then T
   __shared__ cplx s_tau[32];
@@ -587,22 +629,9 @@ __global__ __launch_bounds__(1024) void panel_reg_kernel(cplx* __restrict__ A, i
       for (int t = 0; t < RPL; ++t)
         if (l + 32 * t > j) xs += cabs2(a[t]);
       xs = hsum32(xs);
-      cplx tj = make_double2(0.0, 0.0), sc = make_double2(1.0, 0.0);
-      double beta = alpha.x;
-      if (!(xs == 0.0 && alpha.y == 0.0)) {
-        beta = -copysign(sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xs), alpha.x);
-        const double rb = 1.0 / beta;
-        tj = make_double2((beta - alpha.x) * rb, -alpha.y * rb);
-        // 1 / (alpha - beta) by Smith's scaling with one reciprocal
-        const double zx = alpha.x - beta, zy = alpha.y;
-        if (fabs(zx) >= fabs(zy)) {
-          const double r = zy / zx, id = 1.0 / (zx + r * zy);
-          sc = make_double2(id, -r * id);
-        } else {
-          const double r = zx / zy, id = 1.0 / (zy + r * zx);
-          sc = make_double2(r * id, -id);
-        }
-      }
+      cplx tj, sc;
+      double beta;
+      reflector(alpha, xs, beta, tj, sc);
 #pragma unroll
       for (int t = 0; t < RPL; ++t) {
         const int r = l + 32 * t;
@@ -716,6 +745,224 @@ __global__ __launch_bounds__(1024) void panel_reg_kernel(cplx* __restrict__ A, i
     for (int j = 0; j < ncol; ++j) dd = cmul(dd, csub(make_double2(1.0, 0.0), cscale(s_tau[j], s_vn2[j])));
     pdet[b] = dd;
   }
+}
+
+// ---- panel factorisation in registers for more than 256 rows ------------------------
+// Same contract as panel_reg_kernel.  Lane l of wave w holds rows l, l + 64, ... of the columns w
+// and w + NW, so a column's sums stay inside its wave and one barrier separates two columns, as
+// above.  Every step reads the reflector from LDS once for both of a wave's columns, into
+// registers.  A column left of j adds the Gram entry by the same sum as the others form v^H a, for
+// v is zero above row j and the column holds its own v below.  Y1 = V T^H takes V through LDS in
+// two parts of CH rows (the whole panel would not fit).
+// Bound by the LDS reads of v (NW x rows x 16 bytes a column), the FP64 sums beside them and the
+// chain norm - reflector - LDS - sum of each column.  16 columns of 769 to 1024 rows 83 us, 513 to
+// 768 53 us, 257 to 512 40 us; the LDS kernel, with one column per wave read from and written to
+// LDS twice a step, took 79 us for 8 columns of 1024 rows and 57 for 8 of 576, so that a panel of
+// twice the width also halves the products and launches between panels: G from a new configuration
+// at Ndim 1024 75.1 -> 37 ms, a sweep at Ndim 576 125.7 -> 83.
+// The 256 rows and fewer of the kernel above stay there: its half-waves sum in one step less, and
+// 32 columns take 55 us against 78 here.
+template <int R, int NW>
+__global__ __launch_bounds__(64 * NW) void panel_wave_kernel(cplx* __restrict__ A, int n, int k, int nb,
+                                                            cplx* __restrict__ tau, cplx* __restrict__ Vw,
+                                                            cplx* __restrict__ Y1w, cplx* __restrict__ Tw,
+                                                            cplx* __restrict__ pdet, long long cs) {
+  constexpr int NC = 2 * NW;          // columns
+  constexpr int CH = 64 * R / 2;      // rows of a part of V in LDS
+  A = chain_ptr(A, cs);
+  tau = chain_ptr(tau, cs);
+  Vw = chain_ptr(Vw, cs);
+  Y1w = chain_ptr(Y1w, cs);
+  Tw = chain_ptr(Tw, cs);
+  pdet = chain_ptr(pdet, cs);
+  extern __shared__ cplx smem[];      // loop: v[2][64 R]; afterwards: V[CH x NC], column-major
+  __shared__ cplx s_S[NC * NC];       // Gram above the diagonal, then T
+  __shared__ cplx s_tau[NC];
+  __shared__ double s_vn2[NC];
+  static_assert(2 * 64 * R <= CH * NC && NC <= 64, "the reflectors lie over V; row j < NC is lane j of slot 0");
+  const int tid = threadIdx.x;
+  const int l = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rows = n - k;
+  const int ncol = (k + nb <= n) ? nb : n - k;
+
+  cplx a[2][R];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = wave + NW * i;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = l + 64 * t;
+      a[i][t] = (c < ncol && r < rows) ? A[(k + r) + (long long)(k + c) * n] : make_double2(0.0, 0.0);
+    }
+  }
+  for (int j = 0; j < ncol; ++j) {
+    cplx* const vb = smem + (j & 1) * 64 * R;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (j != wave + NW * i) continue;
+      const cplx alpha = make_double2(__shfl(a[i][0].x, j, 64), __shfl(a[i][0].y, j, 64));
+      double xs = l > j ? cabs2(a[i][0]) : 0.0;
+#pragma unroll
+      for (int t = 1; t < R; ++t) xs += cabs2(a[i][t]);
+      xs = wave_sum(xs);
+      cplx tj, sc;
+      double beta;
+      reflector(alpha, xs, beta, tj, sc);
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        const int r = l + 64 * t;
+        cplx v = make_double2(r == j ? 1.0 : 0.0, 0.0);
+        if (r > j) v = cmul(a[i][t], sc);
+        vb[r] = v;
+        if (r == j) a[i][t] = make_double2(beta, 0.0);
+        else if (r > j) a[i][t] = v;
+      }
+      if (l == 0) {
+        s_tau[j] = tj;
+        tau[k + j] = tj;
+      }
+    }
+    __syncthreads();
+    cplx vr[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) vr[t] = vb[l + 64 * t];
+    const cplx tc = cconj(s_tau[j]);
+    double dx[2] = {0.0, 0.0}, dy[2] = {0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        dx[i] += vr[t].x * a[i][t].x + vr[t].y * a[i][t].y;
+        dy[i] += vr[t].x * a[i][t].y - vr[t].y * a[i][t].x;
+      }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      dx[i] = wave_sum(dx[i]);
+      dy[i] = wave_sum(dy[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int c = wave + NW * i;
+      if (c > j) {
+        // a <- a - conj(tau) v (v^H a)
+        const cplx f = cmul(tc, make_double2(dx[i], dy[i]));
+#pragma unroll
+        for (int t = 0; t < R; ++t) a[i][t] = csub(a[i][t], cmul(f, vr[t]));
+      } else if (c < j && l == 0) {
+        s_S[c + NC * j] = make_double2(dx[i], -dy[i]);   // v_c^H v_j
+      }
+    }
+  }
+  __syncthreads();
+  // columns c of T by a fan-in solve of T^-1 T = 1 from the bottom row up, lane l row l:
+  //   T(i, c) = tau_i (delta_ic - sum_{m > i} S(i, m) T(m, c))
+  cplx tcol[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+  {
+    const cplx tl = l < ncol ? s_tau[l] : make_double2(0.0, 0.0);
+    cplx acc[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+    for (int q = ncol - 1; q >= 0; --q) {
+      const cplx sq = l < q ? s_S[l + NC * q] : make_double2(0.0, 0.0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int c = wave + NW * i;
+        const cplx mine = l <= c ? cmul(tl, make_double2((l == c ? 1.0 : 0.0) - acc[i].x, -acc[i].y)) : make_double2(0.0, 0.0);
+        const cplx tq = make_double2(__shfl(mine.x, q, 64), __shfl(mine.y, q, 64));
+        if (l == q) tcol[i] = tq;
+        acc[i] = cfma(sq, tq, acc[i]);
+      }
+    }
+  }
+  double vn[2] = {0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = wave + NW * i;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = l + 64 * t;
+      const cplx x = a[i][t];
+      cplx v = make_double2(0.0, 0.0);
+      if (c < ncol && r < rows) {
+        v = r > c ? x : make_double2(r == c ? 1.0 : 0.0, 0.0);
+        A[(k + r) + (long long)(k + c) * n] = x;
+        Vw[(k + r) + (long long)(k + c) * n] = v;
+      }
+      a[i][t] = v;
+      vn[i] += cabs2(v);
+    }
+    vn[i] = wave_sum(vn[i]);
+  }
+  __syncthreads();   // the Gram entries and the reflectors are read
+  const int b = k / nb;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = wave + NW * i;
+    if (l < NC) s_S[l + NC * c] = (c < ncol && l < ncol) ? tcol[i] : make_double2(0.0, 0.0);
+    if (c < ncol && l < ncol) Tw[(long long)b * nb * nb + l + c * nb] = tcol[i];
+    if (l == 0) s_vn2[c] = vn[i];
+  }
+  // Y1 = V T^H: Y1(r, j) = sum_{m >= j} V(r, m) conj(T(j, m)), 16 x 16 MFMA tiles
+  const int lr = l & 15, lk = l >> 4;
+  const int tcn = (ncol + 15) / 16, kc = (ncol + 3) & ~3;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (h * CH >= rows) break;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < R / 2; ++t) smem[(l + 64 * t) + CH * (wave + NW * i)] = a[i][h * (R / 2) + t];
+    __syncthreads();
+    const int tr = (rows - h * CH < CH ? rows - h * CH + 15 : CH) / 16;
+    for (int ti = wave; ti < tr * tcn; ti += NW) {
+      const int r0 = 16 * (ti % tr), c0 = 16 * (ti / tr);
+      v4d_t re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+      for (int k0 = c0; k0 < kc; k0 += 4) {
+        const cplx v = smem[(r0 + lr) + CH * (k0 + lk)];
+        const cplx tv = cconj(s_S[(c0 + lr) + NC * (k0 + lk)]);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(tv.x, v.x, re, 0, 0, 0);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(-tv.y, v.y, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(tv.x, v.y, im, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(tv.y, v.x, im, 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = h * CH + r0 + lr, gj = c0 + 4 * q + lk;
+        if (gi < rows && gj < ncol) Y1w[(k + gi) + (long long)(k + gj) * n] = make_double2(re[q], im[q]);
+      }
+    }
+    if (h == 0) __syncthreads();
+  }
+  if (tid == 0) {
+    cplx dd = make_double2(1.0, 0.0);
+    for (int j = 0; j < ncol; ++j) dd = cmul(dd, csub(make_double2(1.0, 0.0), cscale(s_tau[j], s_vn2[j])));
+    pdet[b] = dd;
+  }
+}
+
+template <int RPL>
+int launch_panel_reg(QRWork& w, int k, hipStream_t s) {
+  constexpr size_t lds = (size_t)32 * RPL * 32 * sizeof(cplx);
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [] {
+    attr = hipFuncSetAttribute((const void*)&panel_reg_kernel<RPL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  });
+  HIP_OK(attr);
+  hipLaunchKernelGGL(panel_reg_kernel<RPL>, dim3(1, 1, w.nchain), dim3(1024), lds, s, w.A, w.n, k, w.nb, w.tau, w.Vw,
+                     w.Y1, w.T, w.pdet, w.cs);
+  return ST_NONE;
+}
+template <int R, int NW>
+int launch_panel_wave(QRWork& w, int k, hipStream_t s) {
+  constexpr size_t lds = (size_t)(64 * R / 2) * 2 * NW * sizeof(cplx);
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [] {
+    attr = hipFuncSetAttribute((const void*)&panel_wave_kernel<R, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  });
+  HIP_OK(attr);
+  hipLaunchKernelGGL((panel_wave_kernel<R, NW>), dim3(1, 1, w.nchain), dim3(64 * NW), lds, s, w.A, w.n, k, w.nb, w.tau,
+                     w.Vw, w.Y1, w.T, w.pdet, w.cs);
+  return ST_NONE;
 }
 
 __device__ cplx block_cprod(cplx v, cplx* sh) {
@@ -901,10 +1148,10 @@ inline unsigned nblocks(long long count, int per) { return (unsigned)((count + p
 
 void qr_work_place(QRWork& w, int n, ArenaLayout& ar) {
   w.n = n;
-  // panel width: the widest whose rows x nb panel fits the LDS kernel's 128 KiB
-  if (n <= 256) w.nb = 32;
-  else if (n <= 512) w.nb = 16;
-  else if (n <= 1024) w.nb = 8;
+  // panel width: the widest whose rows x nb panel fits the registers of one workgroup (512 x 32,
+  // 1024 x 16), beyond 1024 rows the LDS kernel's 128 KiB
+  if (n <= 512) w.nb = 32;
+  else if (n <= 1024) w.nb = 16;
   else if (n <= 2048) w.nb = 4;
   else w.nb = 32;
   w.lds_panel = n <= 2048;
@@ -961,16 +1208,20 @@ static int qr_factor(QRWork& w, const cplx* S, int lds, const cplx* D, int ctran
   for (int k = 0; k < n; k += nb) {
     // the register panel takes any panel of at most RP rows (the kernel works on rows k..n-1
     // with leading dimension n), so the later panels of a larger matrix use it too
-    if (n - k <= RP && nb <= 32) {
-      static std::once_flag once_r;
-      static hipError_t attr_r = hipSuccess;
-      std::call_once(once_r, [] {
-        attr_r = hipFuncSetAttribute((const void*)panel_reg_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)(RP * 32 * sizeof(cplx)));
-      });
-      HIP_OK(attr_r);
-      hipLaunchKernelGGL(panel_reg_kernel, dim3(1, 1, w.nchain), dim3(1024), RP * 32 * sizeof(cplx), s, w.A, n, k, nb,
-                         w.tau, w.Vw, w.Y1, w.T, w.pdet, w.cs);
+    const int pr = n - k;
+    if (pr <= RP_MAX && nb <= 32) {
+      st = pr <= 32    ? launch_panel_reg<1>(w, k, s)
+           : pr <= 64  ? launch_panel_reg<2>(w, k, s)
+           : pr <= 128 ? launch_panel_reg<4>(w, k, s)
+                       : launch_panel_reg<8>(w, k, s);
+      if (st) return st;
+    } else if (nb <= 32 && pr <= (nb <= 16 ? 1024 : 512)) {
+      // the fewest rows per lane that hold the panel, as above
+      st = nb > 16     ? (pr <= 384 ? launch_panel_wave<6, 16>(w, k, s) : launch_panel_wave<8, 16>(w, k, s))
+           : pr <= 512 ? launch_panel_wave<8, 8>(w, k, s)
+           : pr <= 768 ? launch_panel_wave<12, 8>(w, k, s)
+                       : launch_panel_wave<16, 8>(w, k, s);
+      if (st) return st;
     } else if (w.lds_panel) {
       const size_t lds = (size_t)(n - k) * std::min(nb, n - k) * sizeof(cplx);
       static std::once_flag once;
