@@ -118,24 +118,23 @@ __global__ void sortperm_kernel(const double* __restrict__ norms, int n, int* __
   perm = chain_ptr(perm, cs);
   pinv = chain_ptr(pinv, cs);
   // four lanes per column j, each counting every fourth i; the lanes' counts are summed with
-  // two exchanges inside the wave, so every lane runs the same number of rounds
-  const int q = threadIdx.x & 3, g = threadIdx.x >> 2, G = blockDim.x >> 2;
-  const int rounds = (n + G - 1) / G;
-  for (int it = 0; it < rounds; ++it) {
-    const int j0 = it * G + g;
-    const int j = j0 < n ? j0 : n - 1;
-    const double x = norms[j];
-    int r = 0;
-    for (int i = q; i < n; i += 4) {
-      const double y = norms[i];
-      r += (y > x) || (y == x && i < j);
-    }
-    r += __shfl_xor(r, 1, 64);
-    r += __shfl_xor(r, 2, 64);
-    if (q == 0 && j0 < n) {
-      perm[r] = j;
-      pinv[j] = r;
-    }
+  // two exchanges inside the wave.  Bound by the loads' latency: the columns are spread over
+  // workgroups and eight loads are in flight per lane
+  const int q = threadIdx.x & 3;
+  const int j0 = blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2);
+  const int j = j0 < n ? j0 : n - 1;
+  const double x = norms[j];
+  int r = 0;
+#pragma unroll 8
+  for (int i = q; i < n; i += 4) {
+    const double y = norms[i];
+    r += (y > x) || (y == x && i < j);
+  }
+  r += __shfl_xor(r, 1, 64);
+  r += __shfl_xor(r, 2, 64);
+  if (q == 0 && j0 < n) {
+    perm[r] = j;
+    pinv[j] = r;
   }
 }
 
@@ -1031,6 +1030,7 @@ __global__ __launch_bounds__(PT) void qr_finish_kernel(const cplx* __restrict__ 
     int odd = 0;
     for (int i = tid; i < n; i += blockDim.x) {
       const int pi = sp[i];
+#pragma unroll 16
       for (int j = i + 1; j < n; ++j) odd ^= (pi > sp[j]) ? 1 : 0;
     }
     if (odd) atomicXor(&s_par, 1);
@@ -1200,7 +1200,7 @@ static int qr_factor(QRWork& w, const cplx* S, int lds, const cplx* D, int ctran
   int st;
   hipLaunchKernelGGL(colnorm_kernel, dim3(nblocks(n, 4), 1, w.nchain), dim3(256), 0, s, S, n, lds, D, ctrans,
                      w.norms, w.cs);
-  hipLaunchKernelGGL(sortperm_kernel, dim3(1, 1, w.nchain), dim3(1024), 0, s, w.norms, n, w.perm, w.pinv, w.cs);
+  hipLaunchKernelGGL(sortperm_kernel, dim3(nblocks(n, 128), 1, w.nchain), dim3(512), 0, s, w.norms, n, w.perm, w.pinv, w.cs);
   hipLaunchKernelGGL(gather_kernel, dim3(nblocks((long long)n * n, 256), 1, w.nchain), dim3(256), 0, s, S, n, lds, D,
                      ctrans, w.perm, w.A, w.cs);
   HIP_OK(hipGetLastError());
