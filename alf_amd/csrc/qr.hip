@@ -758,7 +758,7 @@ __global__ __launch_bounds__(1024) void panel_reg_kernel(cplx* __restrict__ A, i
 // 768 53 us, 257 to 512 40 us; the LDS kernel, with one column per wave read from and written to
 // LDS twice a step, took 79 us for 8 columns of 1024 rows and 57 for 8 of 576, so that a panel of
 // twice the width also halves the products and launches between panels: G from a new configuration
-// at Ndim 1024 75.1 -> 37 ms, a sweep at Ndim 576 125.7 -> 83.
+// at Ndim 1024 75.1 -> 37.5 ms, a sweep at Ndim 576 125.7 -> 80.8.
 // The 256 rows and fewer of the kernel above stay there: its half-waves sum in one step less, and
 // 32 columns take 55 us against 78 here.
 template <int R, int NW>
