@@ -655,7 +655,7 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
             const cplx x = lane_c(xl, js);
             f0 = high && loc == p ? 1.0 : 0.0;
             f1 = high ? make_double2(-1.0, 0.0) : make_double2(-x.x, -x.y);
-            z = lane_c(a.n_sun <= 4 ? zn : renorm_pow2(zn), js);
+            z = lane_c(renorm_pow2(zn), js);
             js_of = lane == mb ? js : js_of;
 #pragma unroll
             for (int i = 0; i < IN; i += 2) {
@@ -703,7 +703,6 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
       };
       if (a.n_sun == 2) decide(std::true_type{});
       else decide(std::false_type{});
-      z = renorm_pow2(z);
       if (lane < mb) {
         const BVisit& w = vc[js_of];
         a.f[(long long)a.slice * a.n_op + (a.dir > 0 ? pos + js_of : a.n_op - 1 - pos - js_of)] = (int8_t)w.fnew;

@@ -1,0 +1,79 @@
+"""Metropolis rounds where a block's own state is at the end of its range, against the oracle's
+sequential visits.
+
+Tolerances: the fields and the random-stream position are the oracle's; G and PHASE to 1e-10, as in
+the other comparisons of whole sweeps (different summation orders in FP64).
+"""
+import cmath
+import math
+
+import numpy as np
+import pytest
+
+from helpers import fields_for, hubbard, oracle, rel
+from oracle.dqmc_oracle import gama, phi
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+
+
+@pytest.fixture(scope="module")
+def rt():
+    from alf_amd import runtime
+    runtime.load_library()
+    return runtime
+
+
+def recorded(s):
+    """Per slice of the oracle's sweeps, the weights |ratio| of its accepted flips."""
+    slices, inner = [], s.upgrade2
+
+    def upgrade2(G, n, nt, new):
+        P, typ, g, E, alpha = s.m.scalars[n]
+        old, g_pp = int(s.f[n, nt]), complex(G[P, P])
+        toggle = inner(G, n, nt, new)
+        if toggle:
+            z1 = g * (phi(new, typ) - phi(old, typ))
+            e = cmath.exp(z1 * E)
+            ratio = (e - (e - 1.0) * g_pp) * cmath.exp(z1 * alpha)
+            slices[-1].append(abs(ratio) ** s.m.n_sun * gama(new, typ) / gama(old, typ))
+        return toggle
+
+    def slice_of(call):
+        def wrap(G, nt):
+            slices.append([])
+            return call(G, nt)
+        return wrap
+
+    s.upgrade2, s.wrapgrup, s.wrapgrdo = upgrade2, slice_of(s.wrapgrup), slice_of(s.wrapgrdo)
+    return slices
+
+
+@pytest.mark.parametrize("n_sun,shift", [(1, 40.0), (2, 20.0), (3, 15.0), (4, 12.0), (5, 9.0)])
+def test_weights_of_a_block_beyond_the_range_of_a_double(rt, n_sun, shift):
+    """A field that couples to a large real shift of the operator: every flip towards the favoured
+    value is taken, with a weight of up to 1e80, so the product of the flips of one block (up to 16
+    of them) is far beyond the largest double while each weight is inside it."""
+    ham = hubbard(L1=5, L2=4, beta=0.6, nwrap=3, U=4.0)
+    ham.N_SUN = n_sun
+    for o in ham.Op_V:
+        o.alpha = 1j * shift
+    f = fields_for(ham, 3)
+    u = np.random.default_rng(7).random(2 * 3 * len(ham.Op_V) * ham.Ltrot + 1)
+    s = oracle(ham, f, u)
+    slices = recorded(s)
+    e = rt.Engine(ham)
+    e.set_fields(f)
+    e.set_tape(u)
+    s.init()
+    e.init()
+    s.sweep()
+    e.sweep(1)
+    assert max(sum(math.log10(r) for r in x[:16]) for x in slices) > 320
+    assert max(r for x in slices for r in x) < 1e150
+    assert np.array_equal(e.get_fields(), s.f)
+    assert e.rng_position() == s.rng.pos
+    assert rel(e.get_green(), s.G) < TOL
+    assert abs(e.get_phase() - s.phase) < TOL
+    e.close()
