@@ -295,17 +295,19 @@ struct alfq_ctx {
   // random numbers
   int rng_mode = 0;                      // 0: none, 1: tape, 2: philox
   double* u = nullptr;                   // uniforms in use: the arena's Philox buffer or a tape
-  double* u_arena = nullptr;             // the arena's Philox buffer (u_cap uniforms per chain)
   double* u_tape = nullptr;              // caller-supplied tape (single chains)
   long long u_cap = 0;
-  long long u_arena_cap = 0;
   long long u_len = 0;
   unsigned long long u_base = 0;
   unsigned long long rng_next = 0;       // host mirror of st->rng_pos
   unsigned long long seed = 0;
   unsigned stream_id = 0;
   long long per_visit_sum = 0;           // uniforms per pass over all ops
-  BVisit* vrec = nullptr;                // visit records of a pass, n_op per slice
+  BVisit* vrec = nullptr;                // visit records of a window of slices, n_op each, or (generic
+                                         // kernel) the window's Philox uniforms in the same place
+  bool sweeping = false;                 // windows of several slices; else one slice at a time
+  int vis_lo = 0, vis_hi = 0;            // slices of the window
+  int vis_dir = 0;                       // the pass it was prepared for (0: none)
   bool multi_op = false;                 // some site has several operators
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   KTimer chain_timer;
@@ -313,7 +315,6 @@ struct alfq_ctx {
   bool round_fusion = true;              // one launch for a round's factors and flush (few chains)
   int* stat_dev = nullptr;               // 3 words per chain read after every sweep
   int* stat_host = nullptr;              // their pinned host copy
-  bool visits_ready = false;             // the visits of the running pass are prepared
   // sweeps replayed as HIP graphs, keyed by the host state they start from
   struct HostState {
     cplx* G; cplx* Gtmp; double* u;
@@ -417,9 +418,22 @@ int fill_uniforms(alfq_ctx* c, long long count) {
   return launch_philox_fill(c->u, c->st, count, c->B, c->cs, c->s);
 }
 
-// What the Metropolis visits of slices [s0, s0 + ns) of a pass need before they start: the block
-// kernel's visit records, or the uniforms of the generic kernel.
-int prepare_visits(alfq_ctx* c, int s0, int ns, int dir) {
+// Slices of a window of visits: half a pass, rounded down.  The records of a whole pass (64 bytes a
+// visit) made a chain of 16 x 16 at Ltrot 100 3 % larger than the uniforms of a sweep did (32 or 48
+// bytes); half a pass makes it no larger.  A window costs one launch: two more a sweep measured nothing
+// (4 x 4, 256 chains: 58.95 and 59.00 ms for ten sweeps), windows of a third 0.5 %.
+int visit_window(int ltrot) { return std::max(1, ltrot / 2); }
+
+// What the Metropolis visits of a slice need before they start: the block kernel's visit records, or
+// the uniforms of the generic kernel.  In a sweep they are prepared for a window of slices of the
+// pass, beginning with this one; a field changes only at its own visit.
+int prepare_visits(alfq_ctx* c, int slice, int dir) {
+  if (c->sweeping && c->vis_dir == dir && slice >= c->vis_lo && slice < c->vis_hi) return ST_NONE;
+  const int win = c->sweeping ? visit_window(c->L) : 1;
+  c->vis_dir = dir;
+  c->vis_lo = dir > 0 ? slice : std::max(0, slice + 1 - win);
+  c->vis_hi = dir > 0 ? std::min(c->L, slice + win) : slice + 1;
+  const int s0 = c->vis_lo, ns = c->vis_hi - c->vis_lo;
   if (c->rng_mode == 0 || chain_max_delay(c->n) < c->K) return fill_uniforms(c, ns * c->per_visit_sum);
   VisitArgs a{};
   a.out = c->vrec; a.st = c->st; a.f = c->f;
@@ -446,7 +460,7 @@ int metropolis_slice(alfq_ctx* c, int slice, int dir) {
   a.cs = c->cs; a.nchain = c->B;
   a.lz = c->lz;
   a.uoff = dir > 0 ? c->uoff_up : c->uoff_dn;
-  a.rec = c->vrec + (long long)slice * c->n_op;
+  a.rec = c->vrec + (long long)(slice - c->vis_lo) * c->n_op;
   a.per = (int)c->per_visit_sum;
   a.multi = c->multi_op ? 1 : 0;
   const int worst = c->n_op / c->K + 1;
@@ -705,7 +719,7 @@ int wrapgrup_dev(alfq_ctx* c, int ntau) {
     if ((st = gemm_c(c, g2))) return st;
   }
   std::swap(c->G, c->Gtmp);
-  if (!c->visits_ready && (st = prepare_visits(c, slice, 1, +1))) return st;
+  if ((st = prepare_visits(c, slice, +1))) return st;
   return metropolis_slice(c, slice, +1);
 }
 
@@ -713,7 +727,7 @@ int wrapgrdo_dev(alfq_ctx* c, int ntau) {
   int st;
   if ((st = hop_ready(c))) return st;
   const int slice = ntau - 1;
-  if (!c->visits_ready && (st = prepare_visits(c, slice, 1, -1))) return st;
+  if ((st = prepare_visits(c, slice, -1))) return st;
   if ((st = metropolis_slice(c, slice, -1))) return st;
   if ((st = launch_dvec(c->f, c->n_op, slice, 1, c->n, c->site_ptr, c->site_ops, c->eexp, c->dv_d, c->dv_dinv,
                         c->dv_dconj, c->B, c->cs, c->s)))
@@ -979,9 +993,10 @@ int init_dev(alfq_ctx* c) {
 
 int sweep_dev(alfq_ctx* c) {
   int st;
-  c->visits_ready = true;
+  c->sweeping = true;
+  c->vis_dir = 0;
   st = sweep_body(c);
-  c->visits_ready = false;
+  c->sweeping = false;
   return st;
 }
 
@@ -1022,7 +1037,6 @@ int sweep_body(alfq_ctx* c) {
   int st;
   const auto& s = c->stab;
   const int L = c->L;
-  if ((st = prepare_visits(c, 0, L, +1))) return st;
   if ((st = udv_reset_dev(c, &c->var_r, 'R'))) return st;
   int nst = 1;
   for (int ntau = 0; ntau < L; ++ntau) {
@@ -1038,7 +1052,6 @@ int sweep_body(alfq_ctx* c) {
     }
     if ((st = measure_dev(c, ntau1))) return st;          // main.F90:757-772
   }
-  if ((st = prepare_visits(c, 0, L, -1))) return st;
   if ((st = udv_reset_dev(c, &c->var_l, 'L'))) return st;
   nst = c->nstm - 1;
   for (int ntau = L; ntau >= 1; --ntau) {
@@ -1317,8 +1330,8 @@ void place_chain(alfq_ctx* c, ArenaLayout& ar, int nslot) {
   c->Xc = ar.take<cplx>(nn);
   c->Yc = ar.take<cplx>(nn);
   c->cscal = ar.take<cplx>(4 * (size_t)n);
-  c->u_arena = ar.take<double>((size_t)std::max<long long>(c->u_cap, 1));
-  c->vrec = ar.take<BVisit>((size_t)no * c->L);
+  static_assert(sizeof(BVisit) >= 3 * sizeof(double), "a visit's record holds its uniforms");
+  c->vrec = ar.take<BVisit>((size_t)no * visit_window(c->L));
   qr_work_place(c->qr, n, ar);
   c->pool.assign(nslot, UDVSlot{});
   for (auto& sl : c->pool) {
@@ -1341,9 +1354,6 @@ size_t chain_arena_bytes(const alfq_model_desc* d) {
   t.t_real = d->t_is_real != 0;
   t.symm = d->expT_half != nullptr;
   t.nstm = (t.L % t.W == 0) ? t.L / t.W : t.L / t.W + 1;
-  long long per = 0;
-  for (int i = 0; i < d->n_op; ++i) per += (d->op_type[i] == 2) ? 3 : 2;
-  t.u_cap = 2LL * t.L * per;
   ArenaLayout sizing;
   place_chain(&t, sizing, t.nstm + 6);
   return (sizing.off + 4095) & ~(size_t)4095;
@@ -1400,7 +1410,7 @@ int create_impl(const alfq_model_desc* descs, int nchain, alfq_ctx** out) {
   c->h_op_site = site;
   c->per_visit_sum = 0;
   for (int i = 0; i < no; ++i) c->per_visit_sum += (typ[i] == 2) ? 3 : 2;
-  c->u_cap = c->u_arena_cap = 2LL * c->L * c->per_visit_sum;
+  c->u_cap = visit_window(c->L) * c->per_visit_sum;
   std::vector<int> up(no + 1, 0), dn(no + 1, 0);
   for (int v = 0; v < no; ++v) {
     up[v + 1] = up[v] + ((typ[v] == 2) ? 3 : 2);
@@ -1440,7 +1450,7 @@ int create_impl(const alfq_model_desc* descs, int nchain, alfq_ctx** out) {
   place_chain(c, ar, nslot);
   c->qr.nchain = nchain;
   c->qr.cs = c->cs;
-  c->u = c->u_arena;
+  c->u = (double*)c->vrec;
   const size_t nn = (size_t)n * n;
   const size_t tsz = c->t_real ? sizeof(double) : sizeof(cplx);
   for (int z = 0; z < nchain; ++z) {
@@ -2201,8 +2211,8 @@ int alfq_rng_set_philox(alfq_ctx* c, uint64_t seed, uint32_t stream) {
   c->rng_next = 0;
   c->u_len = 0;
   c->u_base = 0;
-  c->u = c->u_arena;
-  c->u_cap = c->u_arena_cap;
+  c->u = (double*)c->vrec;
+  c->u_cap = visit_window(c->L) * c->per_visit_sum;
   // the chain's key and stream live in its device state
   ChainState* stc = at(c, c->st);
   const unsigned long long zero = 0;

@@ -27,8 +27,8 @@ struct ChainState {
   int pad2;
 };
 
-// One visit of the block kernel: proposal, table entries and random numbers, prepared for a whole
-// pass (or one slice) by launch_visits.  With Delta = exp(Z1 E) - 1 the single-colour ratio is
+// One visit of the block kernel: proposal, table entries and random numbers, prepared for a window of
+// a pass's slices (or one slice) by launch_visits.  With Delta = exp(Z1 E) - 1 the single-colour ratio is
 // exp(Z1 alpha) (exp(Z1 E) - Delta G(P,P)) = ca - cb G(P,P); the Metropolis test
 // |Re(PHASE ratio^N_SUN Gama(new)/Gama(old))| / |Re(PHASE)| > u becomes
 // |Re(z ratio^N_SUN)| > thr |Re(z)| with thr = u / |Gama ratio| and z any positive
@@ -84,7 +84,7 @@ int launch_chain(const ChainArgs& a, hipStream_t s, KTimer* timer = nullptr);
 // largest delay depth the submatrix block kernel supports (deeper delays use the generic kernel)
 int chain_max_delay(int n);
 // Visit records of slices [s0, s0 + ns) in the order of a pass (dir > 0: ascending slices and
-// operators) into out[slice * n_op + v], the random numbers taken from st->rng_pos on: from u (a
+// operators) into out[(slice - s0) * n_op + v], the random numbers taken from st->rng_pos on: from u (a
 // tape, u[q - st->u_base]) or, with u null, from the chain's Philox stream.  A field changes only at
 // its own visit, so the records of a pass do not depend on its decisions.  Tables, f, st and out
 // per chain; lz as in ChainArgs.

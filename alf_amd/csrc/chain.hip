@@ -151,7 +151,7 @@ __global__ void visit_kernel(VisitArgs a) {
     w.thr = u1 / fabs(a.gama_ratio[ti]);
     w.fnew = (short)s_new;
   }
-  a.out[(long long)slice * a.n_op + v] = w;
+  a.out[(long long)(slice - a.s0) * a.n_op + v] = w;
 }
 
 __global__ __launch_bounds__(256) void chain_kernel(ChainArgs a) {

@@ -1,4 +1,4 @@
-"""Metropolis rounds where a block's own state is at the end of its range, against the oracle's
+"""Metropolis rounds and passes where their own state reaches the end of its range, against the oracle's
 sequential visits.
 
 Tolerances: the fields and the random-stream position are the oracle's; G and PHASE to 1e-10, as in
@@ -77,3 +77,36 @@ def test_weights_of_a_block_beyond_the_range_of_a_double(rt, n_sun, shift):
     assert rel(e.get_green(), s.G) < TOL
     assert abs(e.get_phase() - s.phase) < TOL
     e.close()
+
+
+@pytest.mark.parametrize("ltrot", [1, 2, 3, 4, 5, 7])
+def test_windows_of_visits(rt, ltrot):
+    """The visits of a pass are prepared half of its slices at a time: passes of one window and of
+    several with and without a remainder, from a tape and from the Philox stream, which a delay
+    beyond the block kernel's reads in windows of uniforms and must follow to the same fields."""
+    ham = hubbard(L1=3, L2=4, beta=0.1 * ltrot, nwrap=2, U=4.0)
+    f = fields_for(ham, 4)
+    u = np.random.default_rng(9).random(2 * 2 * 3 * len(ham.Op_V) * ltrot)
+    s = oracle(ham, f, u)
+    s.init()
+    e = rt.Engine(ham, delay=8)
+    e.set_fields(f)
+    e.set_tape(u)
+    e.init()
+    for _ in range(2):
+        s.sweep()
+        e.sweep(1)
+        assert np.array_equal(e.get_fields(), s.f) and e.rng_position() == s.rng.pos
+        assert rel(e.get_green(), s.G) < TOL
+    e.close()
+    got = []
+    for delay in (8, 40):
+        e = rt.Engine(ham, delay=delay)
+        e.set_fields(f)
+        e.set_philox(21, 2)
+        e.init()
+        e.sweep(4)
+        got.append((e.get_fields(), e.rng_position(), e.get_green()))
+        e.close()
+    assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1] == 4 * 2 * 3 * len(ham.Op_V) * ltrot
+    assert rel(got[1][2], got[0][2]) < TOL
