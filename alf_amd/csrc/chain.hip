@@ -368,8 +368,12 @@ __device__ __forceinline__ int here(int v) {
   return v;
 }
 
-// orders LDS accesses in the program; a wave's own LDS operations complete in that order
-__device__ __forceinline__ void lds_order() { __asm__ volatile("" ::: "memory"); }
+// What a wave hands to another through LDS: released before the flag is stored, acquired after it is
+// read, so that the hand-over is ordered in the language and not by the LDS pipeline alone.  The
+// fences name the LDS only: the deciding wave waits for its LDS writes, not for global memory.  One
+// chain's sweep at 16 x 16 with them 61.4 ms, with a bare compiler barrier in their place 61.2.
+__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+__device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
 
 // Bound by the serial chain of decisions: about 1240 clocks from one acceptance to the next (LDS
 // reads of the row and column, their dot product, the test, the ballot), 20 to 32 of them in a
@@ -396,9 +400,8 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
   __shared__ int s_pub[SB_A + 1];
   constexpr int SB_FIN = 0x100;
 
-  // (a wave's LDS operations complete in program order)
   auto publish = [&](int j, int what) {
-    lds_order();
+    lds_release();
     __hip_atomic_store(&s_pub[j], what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
 
@@ -724,7 +727,7 @@ __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {
       int j = 0;
       while (true) {
         const int pub = __hip_atomic_load(&s_pub[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        lds_order();
+        lds_acquire();
         if (pub == 0) {
           __builtin_amdgcn_s_sleep(1);
           continue;
