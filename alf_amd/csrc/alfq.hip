@@ -24,6 +24,7 @@
 #include "../../include/alfq.h"
 #include "alfq_cb.h"
 #include "alfq_chain.h"
+#include "alfq_gemm_rule.h"
 #include "alfq_obs.h"
 #include "alfq_oz.h"
 #include "alfq_qr.h"

@@ -170,10 +170,6 @@ GemmArgs gemm_args(int M, int N, int K, const void* A, int lda, int opA, bool a_
                    const void* B, int ldb, int opB, bool b_cplx, void* C, int ldc,
                    cplx alpha, cplx beta);
 int gemm_launch(const GemmArgs& g, hipStream_t s);
-// Tiling policies a context may pick (its autotuner measures them): 0 the estimate-based
-// default, 1 the 64 x 64 kernel from one tile per CU, 2 never the 64 x 64 kernel, 3 the
-// direct-load kernel up to 512 tiles of 32 x 32.
-constexpr int GEMM_POLICIES = 4;
 // G += X Y^T (all n x n / n x m, column-major, ld n) with the rank m read from *mdev and
 // clamped to kmax <= CHAIN_BLOCK_KMAX, for the nchain chains of a batch (pointers advance by cs bytes).
 int flush_launch(cplx* G, const cplx* X, const cplx* Y, const int* mdev, int n, int kmax, int nchain,

@@ -20,6 +20,7 @@
 //   * QR trailing updates / Q formation / TRMM / CGR products
 #include "alfq_chain.h"
 #include "alfq_common.h"
+#include "alfq_gemm_rule.h"
 
 namespace {
 
@@ -694,7 +695,6 @@ __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, co
       }
 }
 
-inline long long cdivl(long long a, long long b) { return (a + b - 1) / b; }
 inline unsigned gemm_zdim(const GemmArgs& g) {
   return (unsigned)((g.batch > 1 ? g.batch : 1) * (g.nchain > 1 ? g.nchain : 1));
 }
@@ -1126,66 +1126,24 @@ GemmArgs gemm_args(int M, int N, int K, const void* A, int lda, int opA, bool a_
   return g;
 }
 
-// Tile shape with the least estimated time: every SIMD of the 256 CUs holds one wave of a
-// full round, and a wave's time is proportional to the K it covers (K / KS).
-static int gemm_tile_shape(int M, int N, int K, int batch) {
-  const long long b = batch > 1 ? batch : 1;
-  const long long slots = 256LL * 4;
-  struct Opt { int code, ks; long long tm, tn; };
-  const Opt opts[3] = {{0, 1, 32, 32}, {1, 2, 16, 32}, {2, 4, 16, 16}};
-  int best = 0;
-  double best_cost = 0.0;
-  for (int o = 0; o < 3; ++o) {
-    const long long waves = 4 * b * cdivl(M, opts[o].tm) * cdivl(N, opts[o].tn);
-    const double cost = (double)cdivl(waves, slots) * (double)cdivl(K > 0 ? K : 1, 16 * opts[o].ks);
-    if (o == 0 || cost < best_cost) { best = o; best_cost = cost; }
-  }
-  return opts[best].code;
-}
-
-// grid sizes of the tiling policies: direct-load kernel below direct_below tiles of 32 x 32,
-// 64 x 64 kernel from big_from tiles of 64 x 64 (with 3/4 of their area inside the product)
-struct TilePolicy { long long direct_below, big_from; };
-constexpr TilePolicy kTilePolicy[GEMM_POLICIES] = {{256, 512}, {256, 256}, {256, 1LL << 62}, {512, 512}};
-
-static const TilePolicy& tile_policy(const GemmArgs& g) {
-  return kTilePolicy[(g.policy >= 0 && g.policy < GEMM_POLICIES) ? g.policy : 0];
-}
-
-static bool gemm_direct_path(const GemmArgs& g) {
-  return g.M > 0 && g.N > 0 && cdivl(g.M, 32) * cdivl(g.N, 32) * (long long)gemm_zdim(g) < tile_policy(g).direct_below;
-}
-
 int gemm_launch(const GemmArgs& g, hipStream_t s) {
   if (g.M <= 0 || g.N <= 0) return ST_NONE;
   if (gemm_zdim(g) > 65535) { alfq_set_error("gemm_launch: batch too large"); return ST_GENERIC; }
-  const long long b = gemm_zdim(g);
-  if (gemm_direct_path(g)) {
-    // too few 32 x 32 tiles to fill the device: 16 x 16 tiles, K split over up to 8 waves
-    const int ksteps = g.K > 0 ? (g.K + 3) / 4 : 1;
-    if (ksteps >= 32) launch_direct<8>(g, s);
-    else if (ksteps >= 16) launch_direct<4>(g, s);
-    else if (ksteps >= 8) launch_direct<2>(g, s);
-    else launch_direct<1>(g, s);
-    HIP_OK(hipGetLastError());
-    return ST_NONE;
-  }
-  {
-    // two or more 64 x 64 tiles per CU, at least 3/4 of each tile's area inside the product
-    const long long tm = cdivl(g.M, 64), tn = cdivl(g.N, 64);
-    if (tm * tn * b >= tile_policy(g).big_from && 4LL * g.M * g.N >= 3LL * (64 * tm) * (64 * tn) &&
-        tile_kernel_takes(g)) {
-      launch_tile<2, 2>(g, s);
-      HIP_OK(hipGetLastError());
-      return ST_NONE;
+  switch (gemm_kernel_for(g.M, g.N, g.K, gemm_zdim(g), g.policy, tile_kernel_takes(g))) {
+    case GEMM_DIRECT: {
+      const int ksteps = g.K > 0 ? (g.K + 3) / 4 : 1;
+      if (ksteps >= 32) launch_direct<8>(g, s);
+      else if (ksteps >= 16) launch_direct<4>(g, s);
+      else if (ksteps >= 8) launch_direct<2>(g, s);
+      else launch_direct<1>(g, s);
+      break;
     }
-  }
-  switch (gemm_tile_shape(g.M, g.N, g.K, (int)gemm_zdim(g))) {
-    case 0:
+    case GEMM_TILE_64: launch_tile<2, 2>(g, s); break;
+    case GEMM_TILE_32:
       if (tile_kernel_takes(g)) launch_tile<1, 1>(g, s);
       else launch_shape<2, 2>(g, s);
       break;
-    case 1: launch_shape<1, 2>(g, s); break;
+    case GEMM_LDS_16_32: launch_shape<1, 2>(g, s); break;
     default: launch_shape<1, 1>(g, s); break;
   }
   HIP_OK(hipGetLastError());
