@@ -110,3 +110,67 @@ def test_windows_of_visits(rt, ltrot):
         e.close()
     assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1] == 4 * 2 * 3 * len(ham.Op_V) * ltrot
     assert rel(got[1][2], got[0][2]) < TOL
+
+
+@pytest.mark.parametrize("delay,n_sun", [(1, 2), (15, 1), (16, 2), (17, 3), (31, 2), (32, 2), (32, 4), (32, 5)])
+def test_rounds_of_single_operator_sites(rt, delay, n_sun):
+    """One operator per site on a lattice of several blocks: rounds that fill up, flips carried from
+    block to block of a round, blocks cut short by their 16th flip, and (after a first sweep that
+    accepts little) slices that outgrow the rounds planned for them."""
+    ham = hubbard(L1=7, L2=14, beta=0.6, nwrap=3, U=0.6)
+    ham.N_SUN = n_sun
+    f = fields_for(ham, 3)
+    per = 2 * 3 * ham.Ltrot * len(ham.Op_V)
+    u = np.random.default_rng(7).random(3 * per).reshape(-1, 3)
+    u[:per // 3, 2] = 1.0 - 2.0**-40      # the decisions' numbers
+    u[per // 3:, 2] *= 0.2
+    u = u.ravel()
+    s = oracle(ham, f, u)
+    slices = recorded(s)
+    e = rt.Engine(ham, delay=delay)
+    e.set_fields(f)
+    e.set_tape(u)
+    s.init()
+    e.init()
+    most = []
+    for _ in range(3):
+        del slices[:]
+        s.sweep()
+        e.sweep(1)
+        most.append(max(len(x) for x in slices))
+        assert np.array_equal(e.get_fields(), s.f)
+        assert rel(e.get_green(), s.G) < TOL
+        assert abs(e.get_phase() - s.phase) < TOL
+        assert e.rng_position() == s.rng.pos
+    # the largest slice of the first sweep plans the rounds of the second
+    assert min(most) > max(delay, 16) and most[1] > -(-most[0] // delay) * delay
+    c = e.control()
+    assert c["NC_up"] == s.ctrl.NC_up and c["ACC_up"] == s.ctrl.ACC_up
+    e.close()
+
+
+@pytest.mark.parametrize("L1,L2,chains,fusion", [(16, 16, 16, False), (7, 9, 256, True), (17, 16, 12, True)])
+def test_flush_of_a_batch(rt, L1, L2, chains, fusion):
+    """Batches whose 64 x 64 tiles fill the device (16 tiles a chain, one with a remainder, 25 with
+    remainders): the rounds' factors and the batched flush, against the same chains one at a time."""
+    ham = hubbard(L1=L1, L2=L2, beta=0.4, nwrap=2)
+    fs = [fields_for(ham, 20 + z) for z in range(chains)]
+    b = rt.BatchEngine([ham] * chains)
+    b.round_fusion(fusion)
+    for z in range(chains):
+        b.chain(z).set_fields(fs[z])
+        b.set_philox(31, z)
+    b.init()
+    b.sweep(2)
+    for z in (0, chains // 2, chains - 1):
+        e = rt.Engine(ham)
+        e.set_fields(fs[z])
+        e.set_philox(31, z)
+        e.init()
+        e.sweep(2)
+        b.chain(z)
+        assert np.array_equal(b.get_fields(), e.get_fields()) and not np.array_equal(e.get_fields(), fs[z])
+        assert rel(b.get_green(), e.get_green()) < TOL
+        assert abs(b.get_phase() - e.get_phase()) < TOL
+        e.close()
+    b.close()
