@@ -375,12 +375,13 @@ __device__ __forceinline__ int here(int v) {
 __device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
 __device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
 
-// Bound by the serial chain of decisions: about 1240 clocks from one acceptance to the next (LDS
-// reads of the row and column, their dot product, the test, the ballot), 20 to 32 of them in a
-// launch.  Per launch for one chain of 16 x 16 22.8 us, where one rank-1 update of X, Y and g per
-// acceptance took 30.4 (its sweep 74.9 -> 64.5 ms with the flush); for 256 chains of 4 x 4 20.0 ->
-// 14.3 us.  Rounds deeper than 32 lose in the products of a block what they save in launches (one
-// chain's sweep at 40, 48 and 56: +2, +3 and +7 %), and their error grows with the depth.
+// Bound by two serial parts, for one chain of 16 x 16 24.7 us a launch (34.5 where one rank-1 update
+// of X, Y and g was made per acceptance; its sweep 75.1 -> 61.4 ms with the flush), for 256 chains of
+// 4 x 4 12.1 us (20.0).  The decisions: about 1240 clocks (0.52 us) from one acceptance to the next (LDS
+// reads of the row and column, their dot product, the test, the ballot), 22 of them in a launch, so
+// less than half of it.  The starts of its two to three blocks, most of the rest: the gathers of G at
+// the block's sites, two phases of products with a short K and three barriers, overlapped by nothing.
+// Rounds end at 32 flips because the tables do: at 48 they would take more than the LDS's 160 KB.
 // No array of this kernel may leave the registers: one that the compiler moves to LDS by thread
 // costs a read of the launch packet in host memory, 1.6 us and in a batch of 256 chains 8 us.
 __global__ __launch_bounds__(SB_T, 2) void chain_block_kernel(ChainArgs a) {

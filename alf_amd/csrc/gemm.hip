@@ -12,7 +12,9 @@
 // The host picks the tile shape per launch: at Ndim = 256 a 32 x 32 tiling leaves most of
 // the 256 CUs idle, a 16 x 16 tiling with KS = 4 fills them with a quarter of the per-wave K.
 //
-// gemm_tile_kernel takes the same products where the grid fills the device without a K split.
+// gemm_tile_kernel takes the same products where the grid fills the device without a K split; the
+// 32 x 32 tiles here are left to real products, FP32 operands in other orders than N x N and matrices
+// past 32-bit offsets.  alfq_gemm_rule.h holds the choice between the kernels.
 // These kernels carry every dense product of the sweep:
 //   * hopping wraps  G <- D exp(-dtau T) G exp(dtau T) D^-1       (real T: 2 MFMA/step)
 //   * UDV chain      U <- D exp(-dtau T) U,  U <- exp(-dtau T) conj(D) U
@@ -350,8 +352,9 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs g) {
 // The fragments enter the MFMA exchanged (opB as its first operand), so that the 16 lanes of a
 // result row run along a column of C: 256-byte segments instead of 64.
 //
-// 256 chains of n = 256, per launch: real x complex wraps 430 -> 326 us (53 TF/s), complex x complex
-// 572 -> 500 us (51 TF/s of issued products); one product of n = 1024 issues at 61 TF/s.  The
+// 256 chains of n = 256, per launch: real x complex wraps 430 -> 304 us (56 TF/s), with row scales 353
+// and 382 us (49 and 45 TF/s), complex x complex 572 -> 475 us (54 TF/s of issued products), gathered
+// or scaled 515 to 555; one product of n = 1024 issues at 61 TF/s.  The
 // kernel this replaces chose orders, gathers and edges by branches inside the K stage.  128 x 64
 // tiles, three waves per SIMD and K stages of 32 measured the same or slower.
 //
@@ -604,8 +607,11 @@ __global__ __launch_bounds__(NT, 2) void gemm_tile_kernel(GemmArgs g) {
 // workgroup owns a 64 x 64 tile of one chain's G; the tile itself, in the layout of the product,
 // and the first 16 columns of X (for the tile's rows) and Y (for its columns) are requested at
 // the start, the next 16 columns while the ones before them are multiplied, and G is written once.
-// Bound by the traffic of G (2 x 16 n^2 bytes per chain) and, from m ~ 45 on, by the FP64 matrix
-// rate; X Y^T is three real products (3M).
+// Bound by the traffic of G (2 x 16 n^2 bytes per chain): 256 chains of n = 256 take 76 us for 537 MB
+// in full rounds (7.1 TB/s), 60 -> 49 us over the first sweeps of a random start.  X Y^T is three real
+// products (3M) here, where the round's other products are four: with four the error of G over a
+// slice of 16 x 16 is the same (8.6e-15 against 8.8e-15, mean of 16 chains; 1.8e-14 when X came from
+// W = C D^T), for X and Y are of the size of G's columns and nothing large cancels.
 constexpr int FL_T = 64, FL_C = 16;
 __global__ __launch_bounds__(NT, 2) void flush_kernel(cplx* G, const cplx* X, const cplx* Y, const int* mdev,
                                                       int n, int kmax, long long cs) {
@@ -923,7 +929,8 @@ void launch_direct(const GemmArgs& g, hipStream_t s) {
 //   Go = Gi + X Y^T,   X = Gi(:, A) C,   Y = Yhat D,   Yhat(c, j) = delta(c, P_j) - Gi(P_j, c),
 // A = (P_0 .. P_{m-1}) the round's accepted sites, CD the m x m upper triangular C and, from column
 // CHAIN_BLOCK_KMAX on, D, with leading dimension CHAIN_CD_LD, m = *mdev <= CHAIN_BLOCK_KMAX.
-// All products are four real ones: with three, the imaginary parts get the rounding of the real ones.
+// The products of the kernels below are four real ones: with three, the imaginary parts get the
+// rounding of the real ones (flush_kernel says why it may take three).
 constexpr int RF_T = 16, RF_W = (CHAIN_BLOCK_KMAX + 15) / 16, RF_K = 16 * RF_W;
 
 // One wave's 16 rows r0 .. and columns 16 w .. 16 w + 15 of X or (isy) Y: register q of a lane holds

@@ -524,7 +524,7 @@ class Engine:
 
     def round_fusion(self, on=True):
         """One launch per delayed-update round for contexts of fewer than 32 chains (default)
-        or an X-product and a flush launch (alfq_set_round_fusion)."""
+        or a launch for its columns and one for the flush (alfq_set_round_fusion)."""
         self._c(self.lib.alfq_set_round_fusion(self.ctx, int(on)))
 
     def kernel_timing(self, enable=True):
